@@ -414,12 +414,11 @@ def work(case):
 
 
 def tolerance(case):
-    # fp32 sums rounded to bf16 at the end: another order of the sums moves some results to the neighbouring bf16 value
+    # fp32 sums rounded to bf16 at the end: another order of the sums moves a few results to the neighbouring bf16 value
+    # (other split counts: rel up to 7e-6, one value in a thousand by 2^-8 at most)
     if case["kind"] == "step":  # a change of rounding in one layer travels through all that follow
-        return {"rel": 0.02, "max": 0.5}
-    if case["kind"] in ("proj", "mlp"):
-        return {"rel": 5e-3, "max": 0.1}
-    return {"rel": 4e-3, "max": 0.1}
+        return {"rel": 0.01, "max": 0.25}
+    return {"rel": 1e-3, "max": 0.03}
 
 
 # ---------------------------------------------------------------------------------------------- the same in 64 bits
