@@ -97,23 +97,57 @@ int effective_len(int capacity, int max_seq_len) {
   return (max_seq_len > 0 && max_seq_len < capacity) ? max_seq_len : capacity;
 }
 
-// Split count: enough workgroups to give every CU one (cus / units splits), and no chunk longer than kMaxChunk
-// positions even in the longest row (a chunk streams through one workgroup two tiles at a time, so its latency grows
-// with its length), but no split shorter than min_chunk positions. When the whole K+V span of the longest row fits
-// kOneSplitBytes there is one split (the kernels apply the same bound to each row's actual length): the
-// cross-workgroup merge of two or more splits costs about 2 us, more than one workgroup takes to stream 64 KB (cold,
-// B2 16/8: head_dim 128, 128 positions 4.45 against 5.42 us; head_dim 64, 256 positions 4.47 against 5.17; at 128 KB
-// one split is slower: 6.23 against 5.47).
-int default_splits_for(int units, int D, int len, int cus) {
-  constexpr int kMaxChunk = 256;
+// Most splits a default count takes: one workgroup per CU or one split per kMaxChunk positions, whichever is more, but
+// no split shorter than min_chunk positions; one split when the whole K+V span of the longest row fits kOneSplitBytes
+// (the kernels apply the same bound to each row's actual length): the cross-workgroup merge of two or more splits costs
+// about 2 us, more than one workgroup takes to stream 64 KB (cold, B2 16/8: head_dim 128, 128 positions 4.45 against
+// 5.42 us; head_dim 64, 256 positions 4.47 against 5.17; at 128 KB one split is slower: 6.23 against 5.47). The static
+// scratch refuses by this bound, so the sizes it takes do not follow the tuning below.
+constexpr int kMaxChunk = 256;
+
+int most_splits_for(int64_t units, int D, int len, int cus) {
   if ((int64_t)len * 4 * D <= kOneSplitBytes) return 1;
   const int min_chunk = min_chunk_for(D);
-  const int useful = len > 0 ? (len + min_chunk - 1) / min_chunk : 1;
-  int s = (cus + units - 1) / units;
+  const int useful = (len + min_chunk - 1) / min_chunk;
+  int64_t s = (cus + units - 1) / units;
   const int by_len = (len + kMaxChunk - 1) / kMaxChunk;
   if (s < by_len) s = by_len;
   if (s > useful) s = useful;
   if (s > kMaxSplits) s = kMaxSplits;
+  return s < 1 ? 1 : (int)s;
+}
+
+// Split count. A workgroup streams about 25 GB/s however long its chunk, so what counts is the longest queue of chunks
+// on one CU. us per call below: 8 kv heads unless said, G 2, head_dim 128, 28 or 16 calls on their own caches in a graph.
+//   - One round: s = floor(CUs / units). A workgroup more than the CUs doubles the queue of some (3 rows of 2000: 11
+//     splits (264 workgroups) 9.91, 10 8.48; 2 rows of 4096: 16 splits 9.3, 24 10.9, 32 10.2; 2 rows of 32768: 16 splits
+//     42.8, 32 45.5, 128 50.7).
+//   - More than three rows are a server's batch, whose lengths differ: two rounds (or three where they divide the row
+//     better and the merge still reads its partials in one batch) even the CUs out, as long as a chunk keeps kMaxChunk
+//     positions (16 rows of 128..2048: 2 splits 20.7, 4 18.6, 8 19.6; 12: 5 splits 16.1, 8 13.8; 8 of 500..8192: 4 splits
+//     38.6, 8 33.9, 32 34.4; but 16 rows of 512: 2 splits 9.3, 4 9.9). Rows of one length lose little by it (8 x 4096: 4
+//     splits 23.8, 8 25.7, 16 26.3).
+//   - Past kMergeBatch splits the merge takes further batches of partials, so more are used only for chunks of at least
+//     kMaxChunk positions (1 kv head, G 8, 4000 positions: 16 splits 14.7, 32 12.4, 128 19.6; 2 kv heads, G 4, 1000
+//     positions: 16 splits 6.13, 32 6.72).
+//   - Rows of up to twice kOneSplitBytes are not split where the rows alone take half of the CUs (16 rows of 200: 1 split
+//     6.09, 2 7.00; 8 such rows: 5.72, 6.39).
+int default_splits_for(int rows, int NKV, int D, int len, int cus) {
+  constexpr int kMergeBatch = 16, kPairRows = 3;
+  const int64_t units = (int64_t)rows * NKV;
+  if (2 * units >= cus && (int64_t)len * 4 * D <= 2 * kOneSplitBytes) return 1;
+  const int most = most_splits_for(units, D, len, cus), by_len = (len + kMaxChunk - 1) / kMaxChunk;
+  int s = (int)(cus / units);
+  if (rows > kPairRows) {
+    int two = (int)(2 * cus / units);
+    const int three = (int)(3 * cus / units);
+    if (three <= kMergeBatch && 3 * two < 2 * three) two = three;
+    const int longest = s > by_len ? s : by_len;
+    s = two < longest ? two : longest;
+  }
+  const int batch = by_len > kMergeBatch ? by_len : kMergeBatch;
+  if (s > batch) s = batch;
+  if (s > most) s = most;
   return s < 1 ? 1 : s;
 }
 
@@ -158,7 +192,7 @@ int resolve_splits(const bz_gqa_decode_args* a, int* splits) {
   int cus = 0;
   const int rc = device_cus(&cus);
   if (rc != BZ_OK) return rc;
-  *splits = default_splits_for(rows_of(a) * a->num_kv_heads, a->head_dim,
+  *splits = default_splits_for(rows_of(a), a->num_kv_heads, a->head_dim,
                                effective_len(a->capacity, a->max_seq_len), cus);
   return BZ_OK;
 }
@@ -290,10 +324,17 @@ int launch(const bz_gqa_decode_args* a, hipStream_t stream, const int32_t* seq_l
     wsb = static_cast<char*>(a->workspace);
   } else {
     if ((long long)R * NKV > kScratchGroups) return BZ_ERR_SCRATCH;
+    int most = splits;
+    if (a->num_splits == 0) {
+      int cus = 0;
+      rc = device_cus(&cus);
+      if (rc != BZ_OK) return rc;
+      most = most_splits_for((int64_t)R * NKV, D, effective_len(cap, a->max_seq_len), cus);
+    }
     ws.counters = 0;
     ws.ml = (size_t)kScratchGroups * kCounterStride * sizeof(int);
-    ws.acc = align256(ws.ml + (size_t)R * NH * splits * sizeof(float2));
-    ws.total = align256(ws.acc + (size_t)R * NH * splits * D * sizeof(float));
+    ws.acc = align256(ws.ml + (size_t)R * NH * most * sizeof(float2));
+    ws.total = align256(ws.acc + (size_t)R * NH * most * D * sizeof(float));
     if (ws.total > kScratchBytes) return BZ_ERR_SCRATCH;
     wsb = static_cast<char*>(scratch_base);
   }
@@ -527,7 +568,7 @@ __attribute__((visibility("default"))) int bz_gqa_decode_workspace_size(int32_t 
     int cus = 0;
     rc = device_cus(&cus);
     if (rc != BZ_OK) return rc;
-    splits = default_splits_for(batch * num_kv_heads, head_dim, effective_len(capacity, max_seq_len), cus);
+    splits = default_splits_for(batch, num_kv_heads, head_dim, effective_len(capacity, max_seq_len), cus);
   }
   *bytes = ws_layout(batch, num_q_heads, num_kv_heads, head_dim, splits).total;
   return BZ_OK;
@@ -542,7 +583,7 @@ __attribute__((visibility("default"))) int bz_gqa_decode_default_splits(int32_t 
   int cus = 0;
   const int rc = device_cus(&cus);
   if (rc != BZ_OK) return rc;
-  *num_splits = default_splits_for(batch * num_kv_heads, head_dim, effective_len(capacity, max_seq_len), cus);
+  *num_splits = default_splits_for(batch, num_kv_heads, head_dim, effective_len(capacity, max_seq_len), cus);
   return BZ_OK;
 }
 

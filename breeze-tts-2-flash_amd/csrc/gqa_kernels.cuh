@@ -568,7 +568,7 @@ __global__ void __launch_bounds__(NT) gqa_split_kernel(const int32_t* lens, cons
   uint4 xe[NS], we[NS], xv, rc, rs;
   int64_t newpos64 = -1;
   // The row's length and start first, ahead of every vector load of the workgroup: the CU's vector memory queue is
-  // shared with the workgroups already streaming there (four per CU on a 1024-workgroup grid), and a q load waiting
+  // shared with the workgroups already streaming there (two per CU on a 512-workgroup grid), and a q load waiting
   // for room in it would hold up these scalar loads behind it in program order. Their addresses come from the
   // preloaded leading arguments (the range arrays, and the token count that gives the row index), so the loads go
   // out together with those of the argument buffer instead of one round trip after them.
