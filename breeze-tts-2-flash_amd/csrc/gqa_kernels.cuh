@@ -17,7 +17,8 @@
 //   A workgroup streams its chunk in tiles of ROWS * PPT positions, two tiles in flight (ping-pong). A KV row of
 //   head_dim bf16 is read by LPR = head_dim / 8 consecutive lanes, 16 bytes each, so one wave64 load instruction
 //   covers 64 * 16 B of consecutive positions and every K/V byte is read once, by one lane, straight into VGPRs.
-//   All G q heads of the GQA group use the same K/V registers.
+//   All G q heads of the GQA group use the same K/V registers. Groups of 1 and 2 q heads take the vector path described
+//   here, groups of 4 and 8 the matrix cores (use_mfma, WaveTile, consume_wave_tile).
 //   q . k: four v_dot2c_f32_bf16 per head on the packed bf16 words, then a 16- (or 8-) lane DPP row sum.
 //   Softmax: online, base 2 (scale * log2(e) applied to the score), one running max per wave (the rows of a wave
 //   take the tile max across rows with lane swaps), per-row running sums and accumulators. At the end of the chunk
@@ -30,6 +31,8 @@
 #include <hip/hip_runtime.h>
 
 #include <stdint.h>
+
+#include <type_traits>
 
 #include "bz_gqa_decode.h"
 #include "device_common.cuh"
@@ -538,23 +541,205 @@ __device__ __forceinline__ void consume_tile(Tile<PPT>& t, const uint4 (&qp)[G],
   }
 }
 
+// ------------------------------------------------------------------- tiles on the matrix cores (groups of 4 and 8)
+
+constexpr bool use_mfma(int G) { return G >= 4; }
+
+// With four or more q heads per kv head the dot products are a contraction for the matrix cores: the vector path above
+// spends about 70 G VALU instructions per 16 positions and wave (dot2, DPP row sums, an fma per head and dim; at G = 8
+// about 90% of the time the bytes take), while here 16 positions cost 12 MFMAs (20 at G = 8) and about 120 VALU
+// instructions at any G. us per call, vector path against this one, calls on their own caches in a graph: G 8, 2 rows x
+// 4 kv heads x 32768: 43.3 / 28.4 (4.7 TB/s); G 8, 1 x 1 x 4000: 14.7 / 9.2; G 4, D 64, 32 rows of 64..4096: 37.0
+// / 32.0; G 4, 4 x 2 x 2048: 7.6 / 6.7. At G <= 2 the vector path is not the bound and this one measured the same or
+// slower (2 x 8 x 1024: 6.10 either way; 4096: 9.28 / 9.47).
+//
+// One wave's tile of 16 positions in VGPRs. With r = lane % 16 and g = lane / 16:
+//   k[j]  as loaded, 16 bytes of a row each. A load covers 8 rows of 128 bytes (whole cache lines; loading the operand
+//         layout directly, 16 rows of 64 bytes, measured 4-13% slower): load 2 p holds rows 0..7 and load 2 p + 1 rows
+//         8..15, lane (r, g) the row r % 8 (+ 8) and its 16 bytes 128 p + 64 (r / 8) + 16 g. k_operand() trades halves
+//         between lanes r and r ^ 8, so that each lane has its own row r: the dims 32 j + 8 g .. + 7 of position r, the
+//         A operand of K . q^T.
+//   v[i]  dims (D / 16) r .. (D / 16) (r + 1) - 1 of position 4 g + i: the four positions whose scores the lane holds
+//         after K . q^T (MFMA results: column lane % 16, rows 4 g + i), so P goes from the first product to the second
+//         without leaving its lane. A load covers four rows.
+template <int D>
+struct WaveTile {
+  static constexpr int NJ = D / 32;
+  uint4 k[NJ];
+  uint32_t v[4][NJ];
+  float m[4];
+};
+
+// Issue every K and V load of a wave's tile (and its mask values) before any arithmetic; unconditional and non-temporal
+// like load_tile's.
+template <int D, int MK>
+__device__ __forceinline__ void load_wave_tile(WaveTile<D>& t, const Spans& sp, int pos0, int r, int g) {
+  constexpr int NJ = D / 32;
+  const uint32_t koff = (uint32_t)(pos0 + r % 8) * sp.row_bytes + 64 * (r / 8) + 16 * g;
+#pragma unroll
+  for (int j = 0; j < NJ; ++j)
+    t.k[j] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
+                                           sp.k, koff + (j % 2) * 8 * sp.row_bytes + 128 * (j / 2), 0, kStream));
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t pos = (uint32_t)(pos0 + 4 * g + i);
+    const uint32_t voff = pos * sp.row_bytes + (D / 8) * r;
+    if constexpr (D == 128) {
+      const uint4 w = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(sp.v, voff, 0, kStream));
+      t.v[i][0] = w.x, t.v[i][1] = w.y, t.v[i][2] = w.z, t.v[i][3] = w.w;
+    } else {
+      const uint2 w = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(sp.v, voff, 0, kStream));
+      t.v[i][0] = w.x, t.v[i][1] = w.y;
+    }
+    if (MK == BZ_MASK_BF16) t.m[i] = bf16_to_f32(__builtin_amdgcn_raw_buffer_load_b16(sp.m, pos * 2, 0, 0));
+    if (MK == BZ_MASK_F32) t.m[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(sp.m, pos * 4, 0, 0));
+  }
+}
+
+// Lanes r >= 8 of a 16-lane row (BANKS 0xc) or r < 8 (0x3) take x of lane r ^ 8, the others keep `keep`: one DPP move.
+template <int BANKS>
+__device__ __forceinline__ uint32_t trade8(uint32_t keep, uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)keep, (int)x, 0x128, 0xf, BANKS, false);  // row_ror:8
+}
+template <int D>
+__device__ __forceinline__ bf16x8_t k_operand(const WaveTile<D>& t, int j) {
+  const uint4 &a = t.k[j / 2 * 2], &b = t.k[j / 2 * 2 + 1];  // rows 0..7, rows 8..15
+  const uint4 o = j % 2 == 0
+                      ? make_uint4(trade8<0xc>(a.x, b.x), trade8<0xc>(a.y, b.y), trade8<0xc>(a.z, b.z), trade8<0xc>(a.w, b.w))
+                      : make_uint4(trade8<0x3>(b.x, a.x), trade8<0x3>(b.y, a.y), trade8<0x3>(b.z, a.z), trade8<0x3>(b.w, a.w));
+  return __builtin_bit_cast(bf16x8_t, o);
+}
+
+// The bf16 pair (low half of a, low half of b) or (high half of a, high half of b), a first.
+__device__ __forceinline__ uint32_t pair_lo(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x05040100u); }
+__device__ __forceinline__ uint32_t pair_hi(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
+__device__ __forceinline__ float hi16(float x) { return __uint_as_float(__float_as_uint(x) & 0xffff0000u); }
+
+// The running state of one wave. Every lane belongs to q head r % G of the group; lanes of one head hold the same m,
+// and l is summed over the lane's own positions only (the four lane groups are added at the end).
+// P . V keeps p in full fp32: p = hi + mid + lo exactly, three bf16 terms of 8 bits each, whose products are summed by
+// the matrix unit in fp32. For G = 4 the terms sit in columns of the P operand that the heads leave free (columns
+// [0, 4) hold the hi terms of the heads, [4, 8) the mid, [8, 12) the lo terms), so they cost no further products; for
+// G = 8 columns [0, 8) hold hi and [8, 16) mid, and the lo terms take a second product (acc[1]).
+template <int D, int G>
+struct WaveState {
+  static constexpr int NA = G == 8 ? 2 : 1;
+  float m, l;
+  f32x4_t acc[NA][D / 16];  // acc[.][n][i]: dim (D / 16)(4 g + i) + n of column r
+};
+
+// Fold one tile into the running state: K . q^T on the matrix unit (A: positions, B: the q heads repeated over the 16
+// columns), online softmax in base 2 with one max per wave and head, then V^T . P^T. pos0: the tile's first position.
+// A position past hi (or excluded by the mask) is dropped by selects: its score to -inf, and with a mask its V to 0 (a
+// position past hi reads V as 0), so that NaN there reaches nothing. No branch, except for the fused step's new slot
+// (newpos in this tile, uniform over the wave), whose k and v come from registers.
+template <int D, int G, int MK, bool FUSED>
+__device__ __forceinline__ void consume_wave_tile(WaveTile<D>& t, const bf16x8_t (&qf)[D / 32], float scale_log2,
+                                                  WaveState<D, G>& st, int pos0, int r, int g, int hi, int newpos,
+                                                  const uint4 (&knew)[D / 32], const uint4& vnew) {
+  constexpr int NJ = D / 32;
+  bf16x8_t kf[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) kf[j] = k_operand<D>(t, j);
+  if (FUSED && newpos >= pos0 && newpos < pos0 + 16) {
+    const bool fresh = pos0 + r == newpos;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const uint4 k = __builtin_bit_cast(uint4, kf[j]);
+      kf[j] = __builtin_bit_cast(bf16x8_t, make_uint4(fresh ? knew[j].x : k.x, fresh ? knew[j].y : k.y,
+                                                      fresh ? knew[j].z : k.z, fresh ? knew[j].w : k.w));
+    }
+    const uint32_t nv[4] = {vnew.x, vnew.y, vnew.z, vnew.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int w = 0; w < NJ; ++w) t.v[i][w] = pos0 + 4 * g + i == newpos ? nv[w] : t.v[i][w];
+  }
+  f32x4_t d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[j], qf[j], d, 0, 0, 0);
+  float x[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    bool inc = pos0 + 4 * g + i < hi;
+    x[i] = d[i] * scale_log2;
+    if (MK != BZ_MASK_NONE) {
+      inc = inc && t.m[i] > kExcluded;
+      x[i] = fmaf(t.m[i], kLog2e, x[i]);
+#pragma unroll
+      for (int w = 0; w < NJ; ++w) t.v[i][w] = inc ? t.v[i][w] : 0u;
+    }
+    x[i] = inc ? x[i] : -INFINITY;
+  }
+  float mt[1] = {fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]))};
+  rows_max<1>(mt);
+  const float mn = fmaxf(st.m, mt[0]);
+  const float mu = (mn == -INFINITY) ? 0.f : mn;
+  const float alpha = fast_exp2(st.m - mu);
+  st.m = mn;
+  st.l *= alpha;
+#pragma unroll
+  for (int a = 0; a < WaveState<D, G>::NA; ++a)
+#pragma unroll
+    for (int n = 0; n < D / 16; ++n) st.acc[a][n] *= alpha;
+  // this lane's term of each p (see WaveState)
+  const uint32_t m1 = r >= G ? 0xffff0000u : 0u, m2 = r >= 2 * G ? 0xffff0000u : 0u;
+  float ta[4], tl[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float p = fast_exp2(x[i] - mu);
+    st.l += p;
+    if constexpr (G == 8) {
+      const float r1 = p - hi16(p);
+      ta[i] = r >= 8 ? r1 : p;
+      tl[i] = r1 - hi16(r1);
+    } else {
+      const float r1 = p - __uint_as_float(__float_as_uint(p) & m1);
+      ta[i] = r1 - __uint_as_float(__float_as_uint(r1) & m2);
+    }
+  }
+  auto pack = [](const float (&f)[4]) {  // each term is exact in its high 16 bits
+    return __builtin_bit_cast(s16x4_t, make_uint2(pair_hi(__float_as_uint(f[0]), __float_as_uint(f[1])),
+                                                  pair_hi(__float_as_uint(f[2]), __float_as_uint(f[3]))));
+  };
+  const s16x4_t pa = pack(ta);
+#pragma unroll
+  for (int n = 0; n < D / 16; ++n) {
+    uint32_t vt[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const uint32_t a = t.v[2 * h][n / 2], b = t.v[2 * h + 1][n / 2];
+      vt[h] = n % 2 ? pair_hi(a, b) : pair_lo(a, b);
+    }
+    const s16x4_t va = __builtin_bit_cast(s16x4_t, make_uint2(vt[0], vt[1]));
+    st.acc[0][n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(va, pa, st.acc[0][n], 0, 0, 0);
+    if constexpr (G == 8) st.acc[1][n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(va, pack(tl), st.acc[1][n], 0, 0, 0);
+  }
+}
+
 // ---------------------------------------------------------------------------------------------- kernels
 
 // lens, starts: p.seq_lens and p.kv_start again, as leading (preloaded) arguments.
+// MX: the tiles go through the matrix cores (use_mfma). The bound on registers there keeps the accumulators out
+// of AGPRs, which the rescaling would have to move to and fro.
 template <int D, int G, int PPT, int MK, int NT, bool FUSED>
-__global__ void __launch_bounds__(NT) gqa_split_kernel(const int32_t* lens, const int32_t* starts, const int tpr,
-                                                       const Params p) {
-  constexpr int NW = NT / kWave;        // waves per workgroup
-  constexpr int LPR = D / 8;            // lanes per KV row, 16 B (8 bf16) each
-  constexpr int ROWS = NT / LPR;        // KV rows per load instruction across the workgroup
-  constexpr int TP = ROWS * PPT;        // positions per tile
-  constexpr int RPW = kWave / LPR;      // rows per wave
+__global__ void __launch_bounds__(NT, use_mfma(G) ? (D == 128 ? 2 : 3) : 1)
+    gqa_split_kernel(const int32_t* lens, const int32_t* starts, const int tpr, const Params p) {
+  constexpr bool MX = use_mfma(G);
+  constexpr int NW = NT / kWave;               // waves per workgroup
+  constexpr int LPR = D / 8;                   // lanes per KV row, 16 B (8 bf16) each
+  constexpr int ROWS = NT / LPR;               // KV rows per load instruction across the workgroup
+  constexpr int TP = MX ? 16 * NW : ROWS * PPT;  // positions per tile (MX: 16 consecutive ones per wave)
+  constexpr int RPW = kWave / LPR;             // rows per wave
+  constexpr int NJ = D / 32;                   // MX: MFMAs (32 dims each) per 16 positions of K . q^T
   static_assert(D == 64 || D == 128, "head_dim 64 or 128");
 
   const int split = blockIdx.x, h = blockIdx.y, z = blockIdx.z;  // z = row * T + token
   // tpr = p.T, preloaded: T = 1 but in the depth step's two-token first step
   const int b = tpr == 1 ? z : z / tpr, tok = z - b * tpr;
   const int tid = threadIdx.x, c = tid % LPR, r = tid / LPR;
+  const int lane = tid % kWave, w = tid / kWave;
+  const int mr = lane % 16, mg = lane / 16;  // MX: the lane's place in the MFMA operands
 
   // q of the G heads of this group, this lane's 8 dims, issued first, since none of it depends on the row's length.
   // Fused: the prologue's inputs instead. Its NE = G + 1 heads (the G q heads, then the new k) are spread over the
@@ -564,7 +749,7 @@ __global__ void __launch_bounds__(NT) gqa_split_kernel(const int32_t* lens, cons
   constexpr int NS = (NE + RPW - 1) / RPW;
   static_assert(!FUSED || D == 128, "the fused prologue is built for head_dim 128");
   const int rw = (tid % kWave) / LPR;  // row inside the wave
-  uint4 qr[G];
+  uint4 qr[MX ? NJ : G];
   uint4 xe[NS], we[NS], xv, rc, rs;
   int64_t newpos64 = -1;
   // The row's length and start first, ahead of every vector load of the workgroup: the CU's vector memory queue is
@@ -591,6 +776,12 @@ __global__ void __launch_bounds__(NT) gqa_split_kernel(const int32_t* lens, cons
     rc = *reinterpret_cast<const uint4*>(p.cos + (int64_t)b * p.cs_sb + 8 * c);
     rs = *reinterpret_cast<const uint4*>(p.sin + (int64_t)b * p.cs_sb + 8 * c);
     newpos64 = p.cache_pos[0];
+  } else if constexpr (MX) {
+    // the B operand of K . q^T: head mr % G, dims 32 j + 8 mg (16-byte aligned: the host checks q and its strides)
+    const uint16_t* qsrc =
+        p.q + (int64_t)b * p.q_sb + (int64_t)tok * p.q_st + (int64_t)(h * G + mr % G) * p.q_sh + 8 * mg;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) qr[j] = *reinterpret_cast<const uint4*>(qsrc + 32 * j);
   } else {
 #pragma unroll
     for (int g = 0; g < G; ++g) {
@@ -638,9 +829,15 @@ __global__ void __launch_bounds__(NT) gqa_split_kernel(const int32_t* lens, cons
   // q before streaming. Tiles A and B ping-pong without register copies: while one is consumed the other's loads
   // are in flight. Loads of positions >= hi fall outside the spans and make no memory access, so a one-tile chunk
   // issues no extra traffic.
-  Tile<PPT> ta, tb;
-  load_tile<ROWS, PPT, MK>(ta, sp, lo + r);
-  load_tile<ROWS, PPT, MK>(tb, sp, lo + TP + r);
+  std::conditional_t<MX, WaveTile<D>, Tile<PPT>> ta, tb;
+  // first position of this wave (MX, uniform) or of this lane's row in the tile that starts at t0
+  const int mine = MX ? 16 * wave_uniform(w) : r;
+  auto load = [&](auto& t, int t0) {
+    if constexpr (MX) load_wave_tile<D, MK>(t, sp, t0 + mine, mr, mg);
+    else load_tile<ROWS, PPT, MK>(t, sp, t0 + mine);
+  };
+  load(ta, lo);
+  load(tb, lo + TP);
   // keep the machine scheduler from sinking the tile loads below the q / prologue arithmetic (which would make that
   // arithmetic wait for its own inputs before any K/V load is in flight)
   __builtin_amdgcn_sched_barrier(0);
@@ -648,19 +845,33 @@ __global__ void __launch_bounds__(NT) gqa_split_kernel(const int32_t* lens, cons
   // tiles before the q / prologue arithmetic below (chunk >= min_chunk >= 32)
   const int nact = ceil_div_est(max(len, 1), chunk, __builtin_amdgcn_rcpf((float)chunk));
 
-  uint4 qp[G], knew = make_uint4(0, 0, 0, 0), vnew = make_uint4(0, 0, 0, 0);
+  uint4 qp[MX ? NJ : G], knew = make_uint4(0, 0, 0, 0), vnew = make_uint4(0, 0, 0, 0);
+  [[maybe_unused]] uint4 kop[NJ];  // MX: the new k in the operand's layout
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) kop[j] = make_uint4(0, 0, 0, 0);
   int newpos = -1;
   if (FUSED) {
     uint4 ye[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s) ye[s] = norm_rope8<LPR>(xe[s], we[s], rc, rs, p.eps, c);
     static_assert(RPW * LPR == kWave, "a wave holds whole rows");
+    if constexpr (MX) {
+      const int e = mr % G;
 #pragma unroll
-    for (int e = 0; e < NE; ++e) {
-      const uint4 y = lane_fetch4(ye[e / RPW], (e % RPW) * LPR + c);  // head e from lane c of row e % RPW
-      if (e < G) qp[e] = y;
-      else knew = y;
+      for (int j = 0; j < NJ; ++j) {  // dims 32 j + 8 mg of head e: lane 4 j + mg of row e % 4
+        const int from = (e % 4) * 16 + 4 * j + mg;
+        uint4 y = lane_fetch4(ye[0], from);
+        if constexpr (G == 8) {
+          const uint4 y1 = lane_fetch4(ye[1], from);
+          y = make_uint4(e < 4 ? y.x : y1.x, e < 4 ? y.y : y1.y, e < 4 ? y.z : y1.z, e < 4 ? y.w : y1.w);
+        }
+        qp[j] = y;
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < G; ++e) qp[e] = lane_fetch4(ye[e / RPW], (e % RPW) * LPR + c);  // lane c of row e % RPW
     }
+    knew = lane_fetch4(ye[G / RPW], (G % RPW) * LPR + c);
     vnew = xv;
     if (newpos64 >= 0 && newpos64 < p.cap) {
       const int pos = (int)newpos64;
@@ -670,6 +881,10 @@ __global__ void __launch_bounds__(NT) gqa_split_kernel(const int32_t* lens, cons
       const bool owner = in_range ? (pos >= lo && pos < hi_chunk) : (split == 0);
       if (owner) {
         if (in_range) newpos = pos;
+        if constexpr (MX) {
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) kop[j] = lane_fetch4(ye[G / RPW], (G % RPW) * LPR + 4 * j + mg);
+        }
         if (tid < LPR) {
           const int64_t off = (int64_t)b * p.kv_sb + (int64_t)h * p.kv_sh + (int64_t)pos * p.kv_ss + 8 * c;
           *reinterpret_cast<uint4*>(p.k_out + off) = knew;
@@ -679,63 +894,124 @@ __global__ void __launch_bounds__(NT) gqa_split_kernel(const int32_t* lens, cons
     }
   } else {
 #pragma unroll
-    for (int g = 0; g < G; ++g) qp[g] = qr[g];
+    for (int g = 0; g < (MX ? NJ : G); ++g) qp[g] = qr[g];
   }
 
-  float m[G], l[G], acc[G][8];
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    m[g] = -INFINITY;
-    l[g] = 0.f;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc[g][j] = 0.f;
-  }
-
-  for (int t0 = lo; t0 < hi; t0 += 2 * TP) {
-    consume_tile<LPR, ROWS, G, PPT, MK, FUSED>(ta, qp, p.scale_log2, m, l, acc, t0 + r, hi, newpos, knew, vnew);
-    if (t0 + TP >= hi) break;
-    load_tile<ROWS, PPT, MK>(ta, sp, t0 + 2 * TP + r);
-    consume_tile<LPR, ROWS, G, PPT, MK, FUSED>(tb, qp, p.scale_log2, m, l, acc, t0 + TP + r, hi, newpos, knew, vnew);
-    load_tile<ROWS, PPT, MK>(tb, sp, t0 + 3 * TP + r);
-  }
-
-  // merge the RPW rows of each wave (lanes c, c + LPR, c + 2 LPR, ... hold the same dims): the G * 8 accumulators and
-  // G sums, zero-padded to NQ groups of four, are summed across rows transposed, so row r of red[q] holds the wave's
-  // total of value 4 q + r (for head_dim 64 the two 8-lane rows of each 16-lane row are added first)
-  constexpr int NV = 9 * G, NQ = (NV + 3) / 4;
-  float flat[4 * NQ];
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) flat[8 * g + j] = acc[g][j];
-    flat[8 * G + g] = l[g];
-  }
-#pragma unroll
-  for (int v = NV; v < 4 * NQ; ++v) flat[v] = 0.f;
-  if (LPR == 8) {
-#pragma unroll
-    for (int v = 0; v < NV; ++v) flat[v] += lane_xor8(flat[v]);
-  }
-  float red[NQ];
-#pragma unroll
-  for (int q = 0; q < NQ; ++q) red[q] = rows_sum4(flat[4 * q], flat[4 * q + 1], flat[4 * q + 2], flat[4 * q + 3]);
-
-  // merge the NW waves through LDS
-  __shared__ float s_acc[NW][G][D];
+  // The wave merge's LDS: each wave's accumulators, max and sum per head. MX: NC columns per wave, for G = 4 the hi,
+  // mid and lo columns, added by the reader; PD, the stride of a column, keeps its 16-byte stores free of bank
+  // conflicts.
+  constexpr int NC = MX && G < 8 ? 3 * G : G, PD = MX ? D + 4 : D;
+  __shared__ __align__(16) float s_acc[NW][NC][PD];
   __shared__ float s_m[NW][G], s_l[NW][G];
-  const int w = tid / kWave, lane = tid % kWave, row16 = lane / 16;
-  if (lane % 16 < LPR) {
+
+  if constexpr (MX) {
+    WaveState<D, G> st;
+    st.m = -INFINITY;
+    st.l = 0.f;
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-      const int f = 4 * q + row16;
-      if (f < 8 * G) s_acc[w][f / 8][8 * c + f % 8] = red[q];
-      else if (f < NV && c == 0) s_l[w][f - 8 * G] = red[q];
+    for (int a = 0; a < WaveState<D, G>::NA; ++a)
+#pragma unroll
+      for (int n = 0; n < D / 16; ++n) st.acc[a][n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    bf16x8_t qf[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) qf[j] = __builtin_bit_cast(bf16x8_t, qp[j]);
+    auto consume = [&](auto& t, int t0) {
+      consume_wave_tile<D, G, MK, FUSED>(t, qf, p.scale_log2, st, t0 + mine, mr, mg, hi, newpos, kop, vnew);
+    };
+    for (int t0 = lo; t0 < hi; t0 += 2 * TP) {
+      consume(ta, t0);
+      if (t0 + TP >= hi) break;
+      load(ta, t0 + 2 * TP);
+      consume(tb, t0 + TP);
+      load(tb, t0 + 3 * TP);
+    }
+    // The columns are complete over the wave's positions; only l is still one sum per lane group. For G = 8 the mid
+    // column (8 lanes on) and the lo product are added here. A non-finite hi sum is the result: with V infinite, the
+    // mid and lo terms (which may be 0) would add 0 * inf.
+    float y = st.l;
+    swap16(st.l, y);
+    st.l += y;
+    y = st.l;
+    swap32(st.l, y);
+    st.l += y;
+    if constexpr (G == 8) {
+#pragma unroll
+      for (int n = 0; n < D / 16; ++n)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float rest = lane_xor8(st.acc[0][n][i]) + st.acc[1][n][i];
+          st.acc[0][n][i] += __builtin_isfinite(st.acc[0][n][i]) ? rest : 0.f;
+        }
+    }
+    if (mr < NC) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int n = 0; n < D / 16; n += 4)
+          *reinterpret_cast<f32x4_t*>(&s_acc[w][mr][D / 16 * (4 * mg + i) + n]) =
+              f32x4_t{st.acc[0][n][i], st.acc[0][n + 1][i], st.acc[0][n + 2][i], st.acc[0][n + 3][i]};
+      if (mr < G && mg == 0) {
+        s_m[w][mr] = st.m;
+        s_l[w][mr] = st.l;
+      }
+    }
+  } else {
+    float m[G], l[G], acc[G][8];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      m[g] = -INFINITY;
+      l[g] = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) acc[g][j] = 0.f;
+    }
+
+    auto consume = [&](auto& t, int t0) {
+      consume_tile<LPR, ROWS, G, PPT, MK, FUSED>(t, qp, p.scale_log2, m, l, acc, t0 + r, hi, newpos, knew, vnew);
+    };
+    for (int t0 = lo; t0 < hi; t0 += 2 * TP) {
+      consume(ta, t0);
+      if (t0 + TP >= hi) break;
+      load(ta, t0 + 2 * TP);
+      consume(tb, t0 + TP);
+      load(tb, t0 + 3 * TP);
+    }
+
+    // merge the RPW rows of each wave (lanes c, c + LPR, c + 2 LPR, ... hold the same dims): the G * 8 accumulators and
+    // G sums, zero-padded to NQ groups of four, are summed across rows transposed, so row r of red[q] holds the wave's
+    // total of value 4 q + r (for head_dim 64 the two 8-lane rows of each 16-lane row are added first)
+    constexpr int NV = 9 * G, NQ = (NV + 3) / 4;
+    float flat[4 * NQ];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) flat[8 * g + j] = acc[g][j];
+      flat[8 * G + g] = l[g];
+    }
+#pragma unroll
+    for (int v = NV; v < 4 * NQ; ++v) flat[v] = 0.f;
+    if (LPR == 8) {
+#pragma unroll
+      for (int v = 0; v < NV; ++v) flat[v] += lane_xor8(flat[v]);
+    }
+    float red[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) red[q] = rows_sum4(flat[4 * q], flat[4 * q + 1], flat[4 * q + 2], flat[4 * q + 3]);
+
+    const int row16 = lane / 16;
+    if (lane % 16 < LPR) {
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+        const int f = 4 * q + row16;
+        if (f < 8 * G) s_acc[w][f / 8][8 * c + f % 8] = red[q];
+        else if (f < NV && c == 0) s_l[w][f - 8 * G] = red[q];
+      }
+    }
+    if (lane == 0) {
+#pragma unroll
+      for (int g = 0; g < G; ++g) s_m[w][g] = m[g];
     }
   }
-  if (lane == 0) {
-#pragma unroll
-    for (int g = 0; g < G; ++g) s_m[w][g] = m[g];
-  }
+  // merge the NW waves through LDS
   __syncthreads();
   (void)RPW;
 
@@ -749,8 +1025,13 @@ __global__ void __launch_bounds__(NT) gqa_split_kernel(const int32_t* lens, cons
 #pragma unroll
     for (int u = 0; u < NW; ++u) {
       const float e = fast_exp2(s_m[u][g] - mu);
+      float a = s_acc[u][g][d];
+      if constexpr (NC > G) {  // the hi column, then mid and lo (a non-finite hi sum is the result, see above)
+        const float rest = s_acc[u][G + g][d] + s_acc[u][2 * G + g][d];
+        a += __builtin_isfinite(a) ? rest : 0.f;
+      }
       L = fmaf(e, s_l[u][g], L);
-      A = fmaf(e, s_acc[u][g][d], A);
+      A = fmaf(e, a, A);
     }
     if (nact == 1) {
       p.out[(int64_t)b * p.o_sb + (int64_t)tok * p.o_st + (int64_t)hq * p.o_sh + d] =
@@ -914,10 +1195,9 @@ __global__ void __launch_bounds__(kThreads) gqa_probs_kernel(const Params p, flo
 
 template <int D, int G, int MK, int NT, bool FUSED>
 SplitFn pick_ppt(int ppt) {
-  switch (ppt) {
-    case 1: return gqa_split_kernel<D, G, 1, MK, NT, FUSED>;
-    default: return gqa_split_kernel<D, G, 2, MK, NT, FUSED>;
-  }
+  if constexpr (!use_mfma(G))
+    if (ppt == 2) return gqa_split_kernel<D, G, 2, MK, NT, FUSED>;
+  return gqa_split_kernel<D, G, 1, MK, NT, FUSED>;  // the matrix tiles have one form
 }
 
 template <int D, int G, int NT, bool FUSED>
