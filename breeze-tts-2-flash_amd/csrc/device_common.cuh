@@ -75,6 +75,21 @@ __device__ __forceinline__ float row_sum(float x) {
   return x;
 }
 
+// Max over the 16 lanes of a row; every lane gets it.
+__device__ __forceinline__ float row_max16(float x) {
+  x = fmaxf(x, dpp<0xb1>(x));
+  x = fmaxf(x, dpp<0x4e>(x));
+  x = fmaxf(x, dpp<0x141>(x));
+  return fmaxf(x, dpp<0x140>(x));
+}
+
+// f(i, x of lane i of this lane's 16-lane row) for i = 0 .. 15 (DPP row_newbcast, gfx90a and later).
+template <int I = 0, class F>
+__device__ __forceinline__ void row_lanes(float x, F f) {
+  f(I, dpp<0x150 + I>(x));
+  if constexpr (I < 15) row_lanes<I + 1>(x, f);
+}
+
 // Value of lane (lane ^ 8) inside each 16-lane row: DPP row_ror:8, on the VALU.
 __device__ __forceinline__ float lane_xor8(float x) { return dpp<0x128>(x); }
 
@@ -248,10 +263,7 @@ __device__ __forceinline__ Rsrc span_rsrc(const void* base, int bytes) {
 // Reductions over the wave: inside 16-lane rows with DPP (quad_perm x2, half mirror, mirror), then across rows with
 // the permlane swaps. Every lane ends with the same value.
 __device__ __forceinline__ float wave_max(float x) {
-  x = fmaxf(x, dpp<0xb1>(x));
-  x = fmaxf(x, dpp<0x4e>(x));
-  x = fmaxf(x, dpp<0x141>(x));
-  x = fmaxf(x, dpp<0x140>(x));
+  x = row_max16(x);
   float y = x;
   swap16(x, y);  // [x0 x0 x2 x2], [x1 x1 x3 x3]
   x = fmaxf(x, y);

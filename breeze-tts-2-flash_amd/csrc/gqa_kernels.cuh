@@ -231,27 +231,87 @@ __device__ __forceinline__ void st_agent(float* ptr, float v) {
 // tokens per row (p.T; the split kernel has it in an SGPR from the launch, so a row index needs no division at T = 1).
 // The partials of one (row, kv head) are read through buffer resources cut at nact splits, with the sc1 cache policy
 // (bit 4 of the buffer instruction's cache-policy operand on gfx940 and later: the cache behaviour of an agent-scope
-// relaxed atomic load), so every load is unconditional and splits past nact read 0 without a memory access. All loads
-// are issued before anything waits: each thread's first kBatch partials for its kOut (q head, dim) outputs, and the
-// (max, sum) pairs of q head `wave` (one lane per split). Split weights w_s = 2^(m_s - M) / sum_s 2^(m_s - M) l_s are
-// reduced over the wave and stored to LDS zero-padded, so the weighted sum needs no per-split condition.
+// relaxed atomic load), so the loads of a batch of kBatch splits are unconditional and splits past nact read 0 without a
+// memory access.
 // The partials are left in place: each is written before it is read in every call, and only the counters need to
 // start at zero (clearing the partials as well, so that the whole workspace is zero between calls, cost 0.26 us per
 // call at the serving shape and 0.5 us on the ragged batch).
+constexpr int kBatch = 16;
+
+// Groups with more values (G * D) than threads: each thread owns VW consecutive values and reads them in one load per
+// split, the next batch in flight while one is folded by the online log-sum-exp rule; lane i of each 16-lane row works
+// out split i's weight of the batch (an exp2 is quarter rate) and the row takes the weights by DPP broadcast. No LDS and
+// no barrier. us per call, against merge_few's way: G 8, 1 x 1 kv head x 4000 positions 9.2 -> 7.9, 6 x 1 x 8192 at 32
+// splits 12.2 -> 10.2; G 4, 1 x 2 x 1000 5.66 -> 5.43.
 template <int D, int G, int NT>
-__device__ void merge_splits(const Params& p, int z, int h, int nact, int tpr) {
-  constexpr int kBatch = 16;
+__device__ __forceinline__ void merge_many(const Rsrc& racc, const Rsrc& rml, uint16_t* orow, int64_t o_sh, int nact) {
+  constexpr int VW = G * D / NT;
+  static_assert(VW == 2 || VW == 4, "two or four values per thread");
+  const int tid = threadIdx.x, g = VW * tid / D, lane16 = tid % 16;
+  struct Batch {
+    uint2 ml;
+    float v[kBatch][VW];
+  };
+  auto load = [&](Batch& t, int s0) {
+    t.ml = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rml, ((s0 + lane16) * G + g) * 8, 0, kSc1));
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      const uint32_t off = ((s0 + u) * NT + tid) * VW * 4;
+      if constexpr (VW == 4) {
+        const f32x4_t x = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(racc, off, 0, kSc1));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) t.v[u][i] = x[i];
+      } else {
+        const f32x2_t x = __builtin_bit_cast(f32x2_t, __builtin_amdgcn_raw_buffer_load_b64(racc, off, 0, kSc1));
+        t.v[u][0] = x[0], t.v[u][1] = x[1];
+      }
+    }
+  };
+  float m = -INFINITY, l = 0.f, a[VW];
+#pragma unroll
+  for (int i = 0; i < VW; ++i) a[i] = 0.f;
+  auto fold = [&](const Batch& t, int s0) {
+    const float ms = s0 + lane16 < nact ? __uint_as_float(t.ml.x) : -INFINITY;  // sum and values are 0 past nact
+    const float mn = fmaxf(m, row_max16(ms));
+    const float mu = (mn == -INFINITY) ? 0.f : mn;
+    const float alpha = fast_exp2(m - mu), e = fast_exp2(ms - mu);
+    m = mn;
+    l = fmaf(l, alpha, row_sum<16>(e * __uint_as_float(t.ml.y)));
+#pragma unroll
+    for (int i = 0; i < VW; ++i) a[i] *= alpha;
+    row_lanes(e, [&](int u, float w) {
+#pragma unroll
+      for (int i = 0; i < VW; ++i) a[i] = fmaf(w, t.v[u][i], a[i]);
+    });
+  };
+  Batch ta, tb;
+  load(ta, 0);
+  if (nact > kBatch) load(tb, kBatch);
+  fold(ta, 0);
+  for (int s0 = kBatch; s0 < nact; s0 += 2 * kBatch) {
+    if (s0 + kBatch < nact) load(ta, s0 + kBatch);
+    fold(tb, s0);
+    if (s0 + kBatch >= nact) break;
+    if (s0 + 2 * kBatch < nact) load(tb, s0 + 2 * kBatch);
+    fold(ta, s0 + kBatch);
+  }
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+#pragma unroll
+  for (int i = 0; i < VW; ++i) orow[(int64_t)g * o_sh + (VW * tid) % D + i] = f32_to_bf16(a[i] * inv);
+}
+
+// Groups with up to NT values: one value per thread. All loads are issued before anything waits: each thread's first
+// kBatch partials of its (q head, dim), and the (max, sum) pairs of q head `wave` (one lane per split). Split weights
+// w_s = 2^(m_s - M) / sum_s 2^(m_s - M) l_s are reduced over the wave and stored to LDS zero-padded, so the weighted sum
+// needs no per-split condition.
+template <int D, int G, int NT>
+__device__ __forceinline__ void merge_few(const Rsrc& racc, const Rsrc& rml, uint16_t* orow, int64_t o_sh, int nact) {
   constexpr int NW = NT / kWave;
   constexpr int kOut = (G * D + NT - 1) / NT;
   constexpr int kPerLane = kMaxSplits / kWave;
   constexpr int GD = G * D;
   __shared__ __align__(16) float s_w[G][kMaxSplits];
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
-  const int64_t unit = (int64_t)z * p.NKV + h;
-  const Rsrc racc = span_rsrc(p.part_acc + unit * p.splits * GD, nact * GD * 4);
-  const Rsrc rml = span_rsrc(p.part_ml + unit * p.splits * G, nact * G * 8);
-  const int b = tpr == 1 ? z : z / tpr, tok = z - b * tpr;
-  uint16_t* const orow = p.out + (int64_t)b * p.o_sb + (int64_t)tok * p.o_st;
 
   // The (max, sum) pairs of q head wave % G first, by every wave and without a condition (a wave past the group's
   // heads works a head out again and stores nothing): loads complete in issue order, so the split weights are
@@ -324,8 +384,20 @@ __device__ void merge_splits(const Params& p, int z, int h, int nact, int tpr) {
 #pragma unroll
       for (int u = 0; u < kBatch; ++u) a = fmaf(s_w[g][s0 + u], x[u], a);
     }
-    orow[(int64_t)(h * G + g) * p.o_sh + o % D] = f32_to_bf16(a);
+    orow[(int64_t)g * o_sh + o % D] = f32_to_bf16(a);
   }
+}
+
+template <int D, int G, int NT>
+__device__ void merge_splits(const Params& p, int z, int h, int nact, int tpr) {
+  constexpr int GD = G * D;
+  const int64_t unit = (int64_t)z * p.NKV + h;
+  const Rsrc racc = span_rsrc(p.part_acc + unit * p.splits * GD, nact * GD * 4);
+  const Rsrc rml = span_rsrc(p.part_ml + unit * p.splits * G, nact * G * 8);
+  const int b = tpr == 1 ? z : z / tpr, tok = z - b * tpr;
+  uint16_t* const orow = p.out + (int64_t)b * p.o_sb + (int64_t)tok * p.o_st + (int64_t)h * G * p.o_sh;
+  if constexpr (GD > NT) merge_many<D, G, NT>(racc, rml, orow, p.o_sh, nact);
+  else merge_few<D, G, NT>(racc, rml, orow, p.o_sh, nact);
 }
 
 // Blocks of positions with at least one attended position, recorded while a mask row is scanned: bit i of the
@@ -830,14 +902,14 @@ __global__ void __launch_bounds__(NT, use_mfma(G) ? (D == 128 ? 2 : 3) : 1)
   // are in flight. Loads of positions >= hi fall outside the spans and make no memory access, so a one-tile chunk
   // issues no extra traffic.
   std::conditional_t<MX, WaveTile<D>, Tile<PPT>> ta, tb;
-  // first position of this wave (MX, uniform) or of this lane's row in the tile that starts at t0
-  const int mine = MX ? 16 * wave_uniform(w) : r;
-  auto load = [&](auto& t, int t0) {
-    if constexpr (MX) load_wave_tile<D, MK>(t, sp, t0 + mine, mr, mg);
-    else load_tile<ROWS, PPT, MK>(t, sp, t0 + mine);
-  };
-  load(ta, lo);
-  load(tb, lo + TP);
+  [[maybe_unused]] const int w0 = 16 * wave_uniform(w);  // MX: the wave's first position in a tile
+  if constexpr (MX) {
+    load_wave_tile<D, MK>(ta, sp, lo + w0, mr, mg);
+    load_wave_tile<D, MK>(tb, sp, lo + TP + w0, mr, mg);
+  } else {
+    load_tile<ROWS, PPT, MK>(ta, sp, lo + r);
+    load_tile<ROWS, PPT, MK>(tb, sp, lo + TP + r);
+  }
   // keep the machine scheduler from sinking the tile loads below the q / prologue arithmetic (which would make that
   // arithmetic wait for its own inputs before any K/V load is in flight)
   __builtin_amdgcn_sched_barrier(0);
@@ -915,15 +987,12 @@ __global__ void __launch_bounds__(NT, use_mfma(G) ? (D == 128 ? 2 : 3) : 1)
     bf16x8_t qf[NJ];
 #pragma unroll
     for (int j = 0; j < NJ; ++j) qf[j] = __builtin_bit_cast(bf16x8_t, qp[j]);
-    auto consume = [&](auto& t, int t0) {
-      consume_wave_tile<D, G, MK, FUSED>(t, qf, p.scale_log2, st, t0 + mine, mr, mg, hi, newpos, kop, vnew);
-    };
-    for (int t0 = lo; t0 < hi; t0 += 2 * TP) {
-      consume(ta, t0);
-      if (t0 + TP >= hi) break;
-      load(ta, t0 + 2 * TP);
-      consume(tb, t0 + TP);
-      load(tb, t0 + 3 * TP);
+    for (int t0 = lo + w0; t0 - w0 < hi; t0 += 2 * TP) {
+      consume_wave_tile<D, G, MK, FUSED>(ta, qf, p.scale_log2, st, t0, mr, mg, hi, newpos, kop, vnew);
+      if (t0 - w0 + TP >= hi) break;
+      load_wave_tile<D, MK>(ta, sp, t0 + 2 * TP, mr, mg);
+      consume_wave_tile<D, G, MK, FUSED>(tb, qf, p.scale_log2, st, t0 + TP, mr, mg, hi, newpos, kop, vnew);
+      load_wave_tile<D, MK>(tb, sp, t0 + 3 * TP, mr, mg);
     }
     // The columns are complete over the wave's positions; only l is still one sum per lane group. For G = 8 the mid
     // column (8 lanes on) and the lo product are added here. A non-finite hi sum is the result: with V infinite, the
@@ -965,15 +1034,12 @@ __global__ void __launch_bounds__(NT, use_mfma(G) ? (D == 128 ? 2 : 3) : 1)
       for (int j = 0; j < 8; ++j) acc[g][j] = 0.f;
     }
 
-    auto consume = [&](auto& t, int t0) {
-      consume_tile<LPR, ROWS, G, PPT, MK, FUSED>(t, qp, p.scale_log2, m, l, acc, t0 + r, hi, newpos, knew, vnew);
-    };
     for (int t0 = lo; t0 < hi; t0 += 2 * TP) {
-      consume(ta, t0);
+      consume_tile<LPR, ROWS, G, PPT, MK, FUSED>(ta, qp, p.scale_log2, m, l, acc, t0 + r, hi, newpos, knew, vnew);
       if (t0 + TP >= hi) break;
-      load(ta, t0 + 2 * TP);
-      consume(tb, t0 + TP);
-      load(tb, t0 + 3 * TP);
+      load_tile<ROWS, PPT, MK>(ta, sp, t0 + 2 * TP + r);
+      consume_tile<LPR, ROWS, G, PPT, MK, FUSED>(tb, qp, p.scale_log2, m, l, acc, t0 + TP + r, hi, newpos, knew, vnew);
+      load_tile<ROWS, PPT, MK>(tb, sp, t0 + 3 * TP + r);
     }
 
     // merge the RPW rows of each wave (lanes c, c + LPR, c + 2 LPR, ... hold the same dims): the G * 8 accumulators and
@@ -1015,30 +1081,44 @@ __global__ void __launch_bounds__(NT, use_mfma(G) ? (D == 128 ? 2 : 3) : 1)
   __syncthreads();
   (void)RPW;
 
-  for (int o = tid; o < G * D; o += NT) {
+  // PV consecutive values per thread (MX: their partials go out in one 16-byte store)
+  constexpr int PV = MX ? 4 : 1;
+  for (int o = PV * tid; o < G * D; o += PV * NT) {
     const int g = o / D, d = o % D, hq = h * G + g;
     float M = s_m[0][g];
 #pragma unroll
     for (int u = 1; u < NW; ++u) M = fmaxf(M, s_m[u][g]);
     const float mu = (M == -INFINITY) ? 0.f : M;
-    float L = 0.f, A = 0.f;
+    float L = 0.f, A[PV];
+#pragma unroll
+    for (int i = 0; i < PV; ++i) A[i] = 0.f;
 #pragma unroll
     for (int u = 0; u < NW; ++u) {
       const float e = fast_exp2(s_m[u][g] - mu);
-      float a = s_acc[u][g][d];
-      if constexpr (NC > G) {  // the hi column, then mid and lo (a non-finite hi sum is the result, see above)
-        const float rest = s_acc[u][G + g][d] + s_acc[u][2 * G + g][d];
-        a += __builtin_isfinite(a) ? rest : 0.f;
-      }
       L = fmaf(e, s_l[u][g], L);
-      A = fmaf(e, a, A);
+#pragma unroll
+      for (int i = 0; i < PV; ++i) {
+        float a = s_acc[u][g][d + i];
+        if constexpr (NC > G) {  // the hi column, then mid and lo (a non-finite hi sum is the result, see above)
+          const float rest = s_acc[u][G + g][d + i] + s_acc[u][2 * G + g][d + i];
+          a += __builtin_isfinite(a) ? rest : 0.f;
+        }
+        A[i] = fmaf(e, a, A[i]);
+      }
     }
     if (nact == 1) {
-      p.out[(int64_t)b * p.o_sb + (int64_t)tok * p.o_st + (int64_t)hq * p.o_sh + d] =
-          f32_to_bf16(L > 0.f ? A / L : 0.f);
+      uint16_t* const orow = p.out + (int64_t)b * p.o_sb + (int64_t)tok * p.o_st + (int64_t)hq * p.o_sh + d;
+#pragma unroll
+      for (int i = 0; i < PV; ++i) orow[i] = f32_to_bf16(L > 0.f ? A[i] / L : 0.f);
     } else {
       const int64_t ps = ((int64_t)z * p.NKV + h) * p.splits + split;  // this split of this (row, kv head)
-      st_agent(p.part_acc + ps * (G * D) + o, A);
+      if constexpr (PV == 4) {
+        const Rsrc rp = span_rsrc(p.part_acc + ps * (G * D), G * D * 4);
+        using U4 = decltype(__builtin_amdgcn_raw_buffer_load_b128(rp, 0, 0, 0));
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(U4, f32x4_t{A[0], A[1], A[2], A[3]}), rp, 4 * o, 0, kSc1);
+      } else {
+        st_agent(p.part_acc + ps * (G * D) + o, A[0]);
+      }
       if (d == 0) {
         st_agent(reinterpret_cast<float*>(p.part_ml + ps * G + g), M);
         st_agent(reinterpret_cast<float*>(p.part_ml + ps * G + g) + 1, L);
