@@ -127,14 +127,14 @@ int most_splits_for(int64_t units, int D, int len, int cus) {
 //     positions (16 rows of 128..2048: 2 splits 20.7, 4 18.6, 8 19.6; 12: 5 splits 16.1, 8 13.8; 8 of 500..8192: 4 splits
 //     38.6, 8 33.9, 32 34.4; but 16 rows of 512: 2 splits 9.3, 4 9.9). Rows of one length lose little by it (8 x 4096: 4
 //     splits 23.8, 8 25.7, 16 26.3).
-//   - Past kMergeBatch splits the merge takes further batches of partials, so more are used only for chunks of at least
-//     kMaxChunk positions (1 kv head, G 8, 4000 positions: 16 splits 14.7, 32 12.4, 128 19.6; 2 kv heads, G 4, 1000
-//     positions: 16 splits 6.13, 32 6.72).
+//   - Past kMergeBatch splits the merge takes a second batch of partials: worth it up to two batches for chunks of 32 KB
+//     of K+V (1 row of 2048: 16 splits 6.61, 32 6.28; of 4096: 8.24, 7.50; 2 kv heads, G 4, 1000 positions: 16 splits
+//     5.43, 32 6.03), and beyond for chunks of 128 KB (1 kv head x 8192: 16 splits 10.7, 32 8.0, 256 13.7).
 //   - Rows of up to twice kOneSplitBytes are not split where the rows alone take half of the CUs (16 rows of 200: 1 split
 //     6.09, 2 7.00; 8 such rows: 5.72, 6.39).
 int default_splits_for(int rows, int NKV, int D, int len, int cus) {
   constexpr int kMergeBatch = 16, kPairRows = 3;
-  const int64_t units = (int64_t)rows * NKV;
+  const int64_t units = (int64_t)rows * NKV, kb = (int64_t)len * D / 256;
   if (2 * units >= cus && (int64_t)len * 4 * D <= 2 * kOneSplitBytes) return 1;
   const int most = most_splits_for(units, D, len, cus), by_len = (len + kMaxChunk - 1) / kMaxChunk;
   int s = (int)(cus / units);
@@ -145,8 +145,10 @@ int default_splits_for(int rows, int NKV, int D, int len, int cus) {
     const int longest = s > by_len ? s : by_len;
     s = two < longest ? two : longest;
   }
-  const int batch = by_len > kMergeBatch ? by_len : kMergeBatch;
-  if (s > batch) s = batch;
+  int merged = kb / 32 < 2 * kMergeBatch ? (int)(kb / 32) : 2 * kMergeBatch;
+  if (merged < kMergeBatch) merged = kMergeBatch;
+  if (merged < (kb + 127) / 128) merged = (int)((kb + 127) / 128);
+  if (s > merged) s = merged;
   if (s > most) s = most;
   return s < 1 ? 1 : s;
 }

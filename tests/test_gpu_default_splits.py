@@ -14,8 +14,11 @@ pytestmark = pytest.mark.gpu
 CASES = [
     (2, 16, 8, 128, 2048, 16),    # one round: 256 workgroups
     (3, 16, 8, 128, 2000, 10),    # one round, rounded down: 240
-    (1, 8, 1, 128, 4000, 16),     # the merge batch bounds a single unit
-    (1, 8, 1, 128, 8192, 32),     # ... and chunks of 256 positions where the row is long
+    (1, 8, 1, 128, 1000, 16),     # the merge batch bounds a single unit
+    (1, 8, 1, 128, 1300, 20),     # ... a second batch for chunks of 64 positions
+    (1, 8, 1, 128, 4000, 32),     # ... two batches
+    (1, 8, 1, 128, 9000, 36),     # ... more for chunks of 256 positions
+    (1, 8, 1, 64, 9000, 32),      # (512 at head_dim 64)
     (4, 16, 8, 128, 1024, 8),     # a batch of short rows stays at one round
     (16, 16, 8, 128, 2048, 4),    # two rounds
     (12, 8, 8, 64, 2048, 8),      # three rounds divide the row better
