@@ -231,8 +231,8 @@ __device__ __forceinline__ void st_agent(float* ptr, float v) {
 // tokens per row (p.T; the split kernel has it in an SGPR from the launch, so a row index needs no division at T = 1).
 // The partials of one (row, kv head) are read through buffer resources cut at nact splits, with the sc1 cache policy
 // (bit 4 of the buffer instruction's cache-policy operand on gfx940 and later: the cache behaviour of an agent-scope
-// relaxed atomic load), so the loads of a batch of kBatch splits are unconditional and splits past nact read 0 without a
-// memory access.
+// relaxed atomic load), so the loads of a batch of kBatch splits are unconditional and splits past nact read 0 without
+// a memory access.
 // The partials are left in place: each is written before it is read in every call, and only the counters need to
 // start at zero (clearing the partials as well, so that the whole workspace is zero between calls, cost 0.26 us per
 // call at the serving shape and 0.5 us on the ragged batch).
@@ -240,8 +240,8 @@ constexpr int kBatch = 16;
 
 // Groups with more values (G * D) than threads: each thread owns VW consecutive values and reads them in one load per
 // split, the next batch in flight while one is folded by the online log-sum-exp rule; lane i of each 16-lane row works
-// out split i's weight of the batch (an exp2 is quarter rate) and the row takes the weights by DPP broadcast. No LDS and
-// no barrier. us per call, against merge_few's way: G 8, 1 x 1 kv head x 4000 positions 9.2 -> 7.9, 6 x 1 x 8192 at 32
+// out split i's weight of the batch (an exp2 is quarter rate) and the row takes the weights by DPP broadcast, without
+// LDS or barrier. us per call, against merge_few's way: G 8, 1 x 1 kv head x 4000 positions 9.2 -> 7.9, 6 x 1 x 8192 at 32
 // splits 12.2 -> 10.2; G 4, 1 x 2 x 1000 5.66 -> 5.43.
 template <int D, int G, int NT>
 __device__ __forceinline__ void merge_many(const Rsrc& racc, const Rsrc& rml, uint16_t* orow, int64_t o_sh, int nact) {
@@ -302,8 +302,8 @@ __device__ __forceinline__ void merge_many(const Rsrc& racc, const Rsrc& rml, ui
 
 // Groups with up to NT values: one value per thread. All loads are issued before anything waits: each thread's first
 // kBatch partials of its (q head, dim), and the (max, sum) pairs of q head `wave` (one lane per split). Split weights
-// w_s = 2^(m_s - M) / sum_s 2^(m_s - M) l_s are reduced over the wave and stored to LDS zero-padded, so the weighted sum
-// needs no per-split condition.
+// w_s = 2^(m_s - M) / sum_s 2^(m_s - M) l_s are reduced over the wave and stored to LDS zero-padded, so the weighted
+// sum needs no per-split condition.
 template <int D, int G, int NT>
 __device__ __forceinline__ void merge_few(const Rsrc& racc, const Rsrc& rml, uint16_t* orow, int64_t o_sh, int nact) {
   constexpr int NW = NT / kWave;
@@ -417,53 +417,111 @@ __device__ __forceinline__ bool any_valid(const uint32_t* bits, int shift, int l
   return false;
 }
 
-// [start, end) of mask row b: the first and last position below capacity whose mask value is > -1e30, or [0, 0) if
-// there is none (what mask_range_kernel computes, and bz_mask_interval returns). All NT threads of the workgroup
-// take part, and all get the result. With bits (kValidWords words of LDS), the blocks holding attended positions are
-// recorded there too (valid_shift(cap)), so a workgroup can skip a chunk the mask excludes entirely, as the
-// reference skips its fully masked 64-position chunks (bb_attn.cu:9-11, :151-154).
+// One wave's part of a mask scan: `keep` bit i of lane l stands for position first + VPL * l + i (VPL consecutive
+// positions per lane). lo and hi, uniform over the wave, take in the first and last kept position (ballots and scalar
+// bit counts; a butterfly of min / max over the lanes took twelve LDS permutes), and the 64-position blocks that hold
+// one are recorded in bits (blocks of 1 << shift positions).
+template <int VPL>
+__device__ __forceinline__ void mask_note(uint32_t keep, int first, int lane, int shift, int& lo, int& hi,
+                                          uint32_t* bits) {
+  const uint64_t any = __ballot(keep != 0);
+  if (any == 0) return;
+  const int f = __builtin_ctzll(any), t = 63 - __builtin_clzll(any);
+  const uint32_t kf = (uint32_t)__builtin_amdgcn_readlane((int)keep, f);
+  const uint32_t kt = (uint32_t)__builtin_amdgcn_readlane((int)keep, t);
+  lo = min(lo, first + VPL * f + __builtin_ctz(kf));
+  hi = max(hi, first + VPL * t + 31 - __builtin_clz(kt));
+  if (bits == nullptr) return;
+  constexpr int LPB = 64 / VPL;  // lanes per block of 64 positions; first is a multiple of 64 * VPL
+  if (lane < VPL && ((any >> (LPB * lane % 64)) & (LPB == 64 ? ~0ull : (1ull << (LPB % 64)) - 1)) != 0) {
+    const int blk = (first + 64 * lane) >> shift;
+    atomicOr(&bits[blk >> 5], 1u << (blk & 31));
+  }
+}
+
+// [start, end) of a mask row: the first and last position below cap whose mask value is > -1e30, or [0, 0) if there is
+// none (what bz_mask_interval returns). All NT threads of the workgroup take part, and all get the result. With bits
+// (kValidWords words of LDS), the blocks holding attended positions are recorded there too (valid_shift(cap)), so a
+// workgroup can skip a chunk the mask excludes entirely, as the reference skips its fully masked 64-position chunks
+// (bb_attn.cu:9-11, :151-154).
+// The scan stands before a workgroup's first K/V load, so it is bound by its round trip. A row whose start is 16-byte
+// aligned is read 16 bytes per lane (one load per thread covers 2048 bf16 positions), its last cap % VPL positions and
+// any other row value by value, 8 loads per thread in flight. The row goes through a buffer resource cut at cap: every
+// load is unconditional, and loads past it read 0 and touch no memory. Fused step, B2, 1377 of 2048 slots, bf16 mask, us
+// per call: 8.68 with 2-byte loads and lane butterflies, 8.15 so (6.5 with the range from seq_lens at 1024).
 template <int NT, int MK>
-__device__ void mask_row_range_t(const Params& p, int b, int& start, int& end, uint32_t* bits) {
-  constexpr int kUnroll = 8;  // mask values per thread loaded before any is compared: one round trip per 8 NT
+__device__ void mask_row_range_t(const void* row, int cap, int& start, int& end, uint32_t* bits) {
+  constexpr int kBytes = MK == BZ_MASK_BF16 ? 2 : 4, VPL = 16 / kBytes;
   __shared__ int s_lo[NT / kWave], s_hi[NT / kWave];
-  const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
-  const int shift = valid_shift(p.cap);
-  if (bits != nullptr) {
+  const int tid = threadIdx.x, lane = tid % kWave, wave = wave_uniform(tid / kWave);
+  const int shift = valid_shift(cap);
+  const Rsrc rm = span_rsrc(row, cap * kBytes);
+  auto value = [&](int pos) {
+    return MK == BZ_MASK_BF16 ? bf16_to_f32(__builtin_amdgcn_raw_buffer_load_b16(rm, (uint32_t)pos * kBytes, 0, 0))
+                              : __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rm, (uint32_t)pos * kBytes, 0, 0));
+  };
+  auto clear = [&] {  // after the first loads are issued
+    if (bits == nullptr) return;
     for (int i = tid; i < kValidWords; i += NT) bits[i] = 0;
     __syncthreads();
-  }
-  // the row through a buffer resource cut at the capacity: every load is unconditional (loads past it read 0 and
-  // touch no memory), so the compiler issues the kUnroll loads together
-  constexpr int kBytes = MK == BZ_MASK_BF16 ? 2 : 4;
-  const Rsrc rm = span_rsrc(static_cast<const char*>(p.mask) + (int64_t)b * p.m_sb * kBytes, p.cap * kBytes);
-  int lo = p.cap, hi = -1;
-  for (int base = 0; base < p.cap; base += kUnroll * NT) {
-    float m[kUnroll];
+  };
+  int lo = cap, hi = -1;
+  // kU batches of one position per lane, NT positions apart, from base; positions past cap (or below from) do not count
+  auto singles = [&](auto ku, int base, bool first) {
+    constexpr int kU = decltype(ku)::value;
+    float m[kU];
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-      const uint32_t off = (uint32_t)(base + u * NT + tid) * kBytes;
-      m[u] = MK == BZ_MASK_BF16 ? bf16_to_f32(__builtin_amdgcn_raw_buffer_load_b16(rm, off, 0, 0))
-                                : __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rm, off, 0, 0));
-    }
+    for (int u = 0; u < kU; ++u) m[u] = value(base + u * NT + tid);
+    if (first) clear();
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
+    for (int u = 0; u < kU; ++u) {
       const int pos = base + u * NT + tid;
-      const bool keep = pos < p.cap && m[u] > kExcluded;
-      if (keep) {
-        lo = min(lo, pos);
-        hi = max(hi, pos);
-      }
-      // a wave's 64 positions here are one aligned run of 64, inside one block (shift >= 6): one LDS OR per wave
-      if (bits != nullptr && __ballot(keep) != 0 && lane == 0) {
-        const int blk = (base + u * NT + wave * kWave) >> shift;
-        atomicOr(&bits[blk >> 5], 1u << (blk & 31));
-      }
+      mask_note<1>(pos < cap && m[u] > kExcluded, base + u * NT + wave * kWave, lane, shift, lo, hi, bits);
     }
-  }
+  };
+  // the same for kU loads of VPL positions per lane
+  auto vectors = [&](auto ku, int base, int whole, bool first) {
+    constexpr int kU = decltype(ku)::value;
+    uint4 w[kU];
 #pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) {
-    lo = min(lo, __shfl_xor(lo, off));
-    hi = max(hi, __shfl_xor(hi, off));
+    for (int u = 0; u < kU; ++u)
+      w[u] = __builtin_bit_cast(
+          uint4, __builtin_amdgcn_raw_buffer_load_b128(rm, (uint32_t)(base + (u * NT + tid) * VPL) * kBytes, 0, 0));
+    if (first) clear();
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      float f[8];
+      if constexpr (MK == BZ_MASK_BF16) {
+        unpack8(w[u], f);
+      } else {
+        f[0] = __uint_as_float(w[u].x), f[1] = __uint_as_float(w[u].y);
+        f[2] = __uint_as_float(w[u].z), f[3] = __uint_as_float(w[u].w);
+      }
+      uint32_t keep = 0;
+#pragma unroll
+      for (int i = 0; i < VPL; ++i) keep |= f[i] > kExcluded ? 1u << i : 0u;
+      if (base + (u * NT + tid) * VPL >= whole) keep = 0;
+      mask_note<VPL>(keep, base + (u * NT + wave * kWave) * VPL, lane, shift, lo, hi, bits);
+    }
+  };
+  if ((reinterpret_cast<uintptr_t>(row) & 15) == 0 && (bits == nullptr || shift == 6)) {
+    const int whole = cap / VPL * VPL;
+    const int pos = whole + lane;  // the last cap % VPL positions: a lane each, by every wave
+    const float rest = value(pos);
+    if (cap <= NT * VPL) {
+      vectors(std::integral_constant<int, 1>{}, 0, whole, true);
+    } else {
+      for (int base = 0; base < whole; base += 4 * NT * VPL)
+        vectors(std::integral_constant<int, 4>{}, base, whole, base == 0);
+    }
+    const uint64_t last = __ballot(pos < cap && rest > kExcluded);
+    if (last != 0) {
+      lo = min(lo, whole + __builtin_ctzll(last));
+      hi = max(hi, whole + 63 - __builtin_clzll(last));
+      if (bits != nullptr && tid == 0) atomicOr(&bits[whole >> 11], 1u << ((whole >> 6) & 31));
+    }
+  } else {
+    for (int base = 0; base < cap; base += 8 * NT) singles(std::integral_constant<int, 8>{}, base, base == 0);
   }
   if (lane == 0) {
     s_lo[wave] = lo;
@@ -485,9 +543,10 @@ __device__ void mask_row_range_t(const Params& p, int b, int& start, int& end, u
 template <int NT, int MK = BZ_MASK_NONE>
 __device__ __forceinline__ void mask_row_range(const Params& p, int b, int& start, int& end, uint32_t* bits = nullptr) {
   if (MK == BZ_MASK_BF16 || (MK == BZ_MASK_NONE && p.mask_kind == BZ_MASK_BF16))
-    mask_row_range_t<NT, BZ_MASK_BF16>(p, b, start, end, bits);
+    mask_row_range_t<NT, BZ_MASK_BF16>(static_cast<const uint16_t*>(p.mask) + (int64_t)b * p.m_sb, p.cap, start, end,
+                                       bits);
   else
-    mask_row_range_t<NT, BZ_MASK_F32>(p, b, start, end, bits);
+    mask_row_range_t<NT, BZ_MASK_F32>(static_cast<const float*>(p.mask) + (int64_t)b * p.m_sb, p.cap, start, end, bits);
 }
 
 // Range of query token t of row b, from seq_lens / kv_start or, when seq_lens is NULL, from the mask row (all NT
@@ -676,9 +735,11 @@ __device__ __forceinline__ uint32_t trade8(uint32_t keep, uint32_t x) {
 template <int D>
 __device__ __forceinline__ bf16x8_t k_operand(const WaveTile<D>& t, int j) {
   const uint4 &a = t.k[j / 2 * 2], &b = t.k[j / 2 * 2 + 1];  // rows 0..7, rows 8..15
-  const uint4 o = j % 2 == 0
-                      ? make_uint4(trade8<0xc>(a.x, b.x), trade8<0xc>(a.y, b.y), trade8<0xc>(a.z, b.z), trade8<0xc>(a.w, b.w))
-                      : make_uint4(trade8<0x3>(b.x, a.x), trade8<0x3>(b.y, a.y), trade8<0x3>(b.z, a.z), trade8<0x3>(b.w, a.w));
+  uint4 o;
+  if (j % 2 == 0)
+    o = make_uint4(trade8<0xc>(a.x, b.x), trade8<0xc>(a.y, b.y), trade8<0xc>(a.z, b.z), trade8<0xc>(a.w, b.w));
+  else
+    o = make_uint4(trade8<0x3>(b.x, a.x), trade8<0x3>(b.y, a.y), trade8<0x3>(b.z, a.z), trade8<0x3>(b.w, a.w));
   return __builtin_bit_cast(bf16x8_t, o);
 }
 
@@ -1115,7 +1176,8 @@ __global__ void __launch_bounds__(NT, use_mfma(G) ? (D == 128 ? 2 : 3) : 1)
       if constexpr (PV == 4) {
         const Rsrc rp = span_rsrc(p.part_acc + ps * (G * D), G * D * 4);
         using U4 = decltype(__builtin_amdgcn_raw_buffer_load_b128(rp, 0, 0, 0));
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(U4, f32x4_t{A[0], A[1], A[2], A[3]}), rp, 4 * o, 0, kSc1);
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(U4, f32x4_t{A[0], A[1], A[2], A[3]}), rp, 4 * o, 0,
+                                               kSc1);
       } else {
         st_agent(p.part_acc + ps * (G * D) + o, A[0]);
       }
@@ -1157,37 +1219,26 @@ __global__ void __launch_bounds__(kThreads) gqa_combine_kernel(const Params p) {
   merge_splits<D, G, kThreads>(p, z, h, nact, p.T);
 }
 
-// Interval of the additive mask row: first and last position with value > -1e30.
+// Interval of each additive mask row: first and last position with value > -1e30.
 template <int MK>
 __global__ void __launch_bounds__(kThreads) mask_range_kernel(const void* mask, int64_t m_sb, int cap,
                                                               int32_t* start, int32_t* end) {
-  const int b = blockIdx.x, tid = threadIdx.x;
-  int lo = cap, hi = -1;
-  for (int pos = tid; pos < cap; pos += kThreads) {
-    if (load_mask<MK>(mask, (int64_t)b * m_sb + pos) > kExcluded) {
-      lo = min(lo, pos);
-      hi = max(hi, pos);
+  constexpr int kBytes = MK == BZ_MASK_BF16 ? 2 : 4, kWindow = 1 << 24;  // positions with 32-bit byte offsets
+  const int b = blockIdx.x;
+  const char* row = static_cast<const char*>(mask) + (int64_t)b * m_sb * kBytes;
+  int lo = 0, hi = 0;
+  for (int64_t w0 = 0; w0 < cap; w0 += kWindow) {
+    int s, e;
+    if (w0 > 0) __syncthreads();  // the previous window's LDS has been read
+    mask_row_range_t<kThreads, MK>(row + w0 * kBytes, (int)min<int64_t>(cap - w0, kWindow), s, e, nullptr);
+    if (e > 0) {
+      if (hi == 0) lo = (int)w0 + s;
+      hi = (int)w0 + e;
     }
   }
-#pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) {
-    lo = min(lo, __shfl_xor(lo, off));
-    hi = max(hi, __shfl_xor(hi, off));
-  }
-  __shared__ int s_lo[kWaves], s_hi[kWaves];
-  if (tid % kWave == 0) {
-    s_lo[tid / kWave] = lo;
-    s_hi[tid / kWave] = hi;
-  }
-  __syncthreads();
-  if (tid == 0) {
-    for (int u = 1; u < kWaves; ++u) {
-      lo = min(lo, s_lo[u]);
-      hi = max(hi, s_hi[u]);
-    }
-    const bool any = hi >= 0;
-    start[b] = any ? lo : 0;
-    end[b] = any ? hi + 1 : 0;
+  if (threadIdx.x == 0) {
+    start[b] = lo;
+    end[b] = hi;
   }
 }
 
