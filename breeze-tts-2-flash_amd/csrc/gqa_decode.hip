@@ -22,11 +22,12 @@ SplitFn pick_split(int D, int G, int mk, int ppt, int nt, bool fused) {
   return nullptr;
 }
 
-CombineFn pick_combine(int D, int G) {
-#define BZ_COMBINE_CASE(DD, GG) \
-  if (D == DD && G == GG) return gqa_combine_kernel<DD, GG>;
-  BZ_COMBINE_CASE(128, 1) BZ_COMBINE_CASE(128, 2) BZ_COMBINE_CASE(128, 4) BZ_COMBINE_CASE(128, 8)
-  BZ_COMBINE_CASE(64, 1) BZ_COMBINE_CASE(64, 2) BZ_COMBINE_CASE(64, 4) BZ_COMBINE_CASE(64, 8)
+CombineFn pick_combine(int D, int G, bool mx) {
+#define BZ_COMBINE_CASE(DD, GG, MM) \
+  if (D == DD && G == GG && mx == MM) return gqa_combine_kernel<DD, GG, MM>;
+  BZ_COMBINE_CASE(128, 1, false) BZ_COMBINE_CASE(128, 2, false) BZ_COMBINE_CASE(128, 4, false)
+  BZ_COMBINE_CASE(128, 4, true) BZ_COMBINE_CASE(128, 8, true)
+  BZ_COMBINE_CASE(64, 1, false) BZ_COMBINE_CASE(64, 2, false) BZ_COMBINE_CASE(64, 4, true) BZ_COMBINE_CASE(64, 8, true)
 #undef BZ_COMBINE_CASE
   return nullptr;
 }
@@ -102,7 +103,7 @@ int effective_len(int capacity, int max_seq_len) {
 // (the kernels apply the same bound to each row's actual length): the cross-workgroup merge of two or more splits costs
 // about 2 us, more than one workgroup takes to stream 64 KB (cold, B2 16/8: head_dim 128, 128 positions 4.45 against
 // 5.42 us; head_dim 64, 256 positions 4.47 against 5.17; at 128 KB one split is slower: 6.23 against 5.47). The static
-// scratch refuses by this bound, so the sizes it takes do not follow the tuning below.
+// scratch refuses by this bound and a workspace is sized for it, so neither follows the tuning below.
 constexpr int kMaxChunk = 256;
 
 int most_splits_for(int64_t units, int D, int len, int cus) {
@@ -185,7 +186,12 @@ int check_sizes(int B, int NH, int NKV, int D, int cap) {
 int tokens_of(const bz_gqa_decode_args* a) { return a->tokens_per_row > 1 ? a->tokens_per_row : 1; }
 int rows_of(const bz_gqa_decode_args* a) { return a->batch * tokens_of(a); }
 
-int resolve_splits(const bz_gqa_decode_args* a, int* splits) {
+// step: a fused call with lengths. Up to kStepRows rows over up to kStepLen positions (a backbone decode step) it keeps
+// most_splits_for, the count it always had: another count changes the order of the sums, which travels through the
+// step's later layers (see use_mfma).
+constexpr int kStepRows = 4, kStepLen = 4096;
+
+int resolve_splits(const bz_gqa_decode_args* a, bool step, int* splits) {
   if (a->num_splits < 0 || a->num_splits > kMaxSplits) return BZ_ERR_SHAPE;
   if (a->num_splits > 0) {
     *splits = a->num_splits;
@@ -194,8 +200,11 @@ int resolve_splits(const bz_gqa_decode_args* a, int* splits) {
   int cus = 0;
   const int rc = device_cus(&cus);
   if (rc != BZ_OK) return rc;
-  *splits = default_splits_for(rows_of(a), a->num_kv_heads, a->head_dim,
-                               effective_len(a->capacity, a->max_seq_len), cus);
+  const int rows = rows_of(a), len = effective_len(a->capacity, a->max_seq_len);
+  if (step && rows <= kStepRows && len <= kStepLen)
+    *splits = most_splits_for((int64_t)rows * a->num_kv_heads, a->head_dim, len, cus);
+  else
+    *splits = default_splits_for(rows, a->num_kv_heads, a->head_dim, len, cus);
   return BZ_OK;
 }
 
@@ -315,7 +324,7 @@ int launch(const bz_gqa_decode_args* a, hipStream_t stream, const int32_t* seq_l
   if (mask_kind == BZ_MASK_NONE && seq_lens == nullptr) return BZ_ERR_NULL;
   if (seq_lens != nullptr && wave_route(a, mask_kind, f)) return launch_wave(a, stream, seq_lens, kv_start);
   int splits = 0;
-  int rc = resolve_splits(a, &splits);
+  int rc = resolve_splits(a, f != nullptr && mask_kind == BZ_MASK_NONE, &splits);
   if (rc != BZ_OK) return rc;
   WsLayout ws;
   char* wsb = nullptr;
@@ -348,7 +357,7 @@ int launch(const bz_gqa_decode_args* a, hipStream_t stream, const int32_t* seq_l
   const int nt = kSplitThreads;
   const int ppt = ppt_for(D, G, chunk, nt);
   SplitFn split_fn = pick_split(D, G, mask_kind, ppt, nt, f != nullptr);
-  CombineFn comb_fn = pick_combine(D, G);
+  CombineFn comb_fn = pick_combine(D, G, use_mfma(G, mask_kind, f != nullptr));
   if (split_fn == nullptr || comb_fn == nullptr) return BZ_ERR_UNSUPPORTED;
   // One launch needs no residency of the whole grid: no workgroup waits for another (the last to count in merges,
   // the others leave), so grids larger than the device runs at once merge in the same launch.
@@ -570,7 +579,8 @@ __attribute__((visibility("default"))) int bz_gqa_decode_workspace_size(int32_t 
     int cus = 0;
     rc = device_cus(&cus);
     if (rc != BZ_OK) return rc;
-    splits = default_splits_for(batch, num_kv_heads, head_dim, effective_len(capacity, max_seq_len), cus);
+    // of every default count (a fused step's can be higher than bz_gqa_decode's)
+    splits = most_splits_for((int64_t)batch * num_kv_heads, head_dim, effective_len(capacity, max_seq_len), cus);
   }
   *bytes = ws_layout(batch, num_q_heads, num_kv_heads, head_dim, splits).total;
   return BZ_OK;

@@ -238,7 +238,7 @@ __device__ __forceinline__ void st_agent(float* ptr, float v) {
 // call at the serving shape and 0.5 us on the ragged batch).
 constexpr int kBatch = 16;
 
-// Groups with more values (G * D) than threads: each thread owns VW consecutive values and reads them in one load per
+// Matrix tiles with more values (G * D) than threads: each thread owns VW consecutive values and reads them in one load per
 // split, the next batch in flight while one is folded by the online log-sum-exp rule; lane i of each 16-lane row works
 // out split i's weight of the batch (an exp2 is quarter rate) and the row takes the weights by DPP broadcast, without
 // LDS or barrier. us per call, against merge_few's way: G 8, 1 x 1 kv head x 4000 positions 9.2 -> 7.9, 6 x 1 x 8192 at 32
@@ -300,7 +300,7 @@ __device__ __forceinline__ void merge_many(const Rsrc& racc, const Rsrc& rml, ui
   for (int i = 0; i < VW; ++i) orow[(int64_t)g * o_sh + (VW * tid) % D + i] = f32_to_bf16(a[i] * inv);
 }
 
-// Groups with up to NT values: one value per thread. All loads are issued before anything waits: each thread's first
+// Every other merge: one value per thread at a time. All loads are issued before anything waits: each thread's first
 // kBatch partials of its (q head, dim), and the (max, sum) pairs of q head `wave` (one lane per split). Split weights
 // w_s = 2^(m_s - M) / sum_s 2^(m_s - M) l_s are reduced over the wave and stored to LDS zero-padded, so the weighted
 // sum needs no per-split condition.
@@ -388,7 +388,8 @@ __device__ __forceinline__ void merge_few(const Rsrc& racc, const Rsrc& rml, uin
   }
 }
 
-template <int D, int G, int NT>
+// MX: the partials come from the matrix tiles (the vector path's merge stays what it was, with its bits).
+template <int D, int G, int NT, bool MX>
 __device__ void merge_splits(const Params& p, int z, int h, int nact, int tpr) {
   constexpr int GD = G * D;
   const int64_t unit = (int64_t)z * p.NKV + h;
@@ -396,7 +397,7 @@ __device__ void merge_splits(const Params& p, int z, int h, int nact, int tpr) {
   const Rsrc rml = span_rsrc(p.part_ml + unit * p.splits * G, nact * G * 8);
   const int b = tpr == 1 ? z : z / tpr, tok = z - b * tpr;
   uint16_t* const orow = p.out + (int64_t)b * p.o_sb + (int64_t)tok * p.o_st + (int64_t)h * G * p.o_sh;
-  if constexpr (GD > NT) merge_many<D, G, NT>(racc, rml, orow, p.o_sh, nact);
+  if constexpr (MX && GD > NT) merge_many<D, G, NT>(racc, rml, orow, p.o_sh, nact);
   else merge_few<D, G, NT>(racc, rml, orow, p.o_sh, nact);
 }
 
@@ -674,7 +675,10 @@ __device__ __forceinline__ void consume_tile(Tile<PPT>& t, const uint4 (&qp)[G],
 
 // ------------------------------------------------------------------- tiles on the matrix cores (groups of 4 and 8)
 
-constexpr bool use_mfma(int G) { return G >= 4; }
+// Groups of 8 always; groups of 4 but in the fused step with lengths (the backbone's decode step): a difference of
+// rounding in one layer's attention travels through every later layer of a step (28 layers: 1.7% in the logits from 1e-5 in
+// each call), and a step's results stay what they were, bit for bit.
+constexpr bool use_mfma(int G, int MK, bool FUSED) { return G == 8 || (G == 4 && !(FUSED && MK == BZ_MASK_NONE)); }
 
 // With four or more q heads per kv head the dot products are a contraction for the matrix cores: the vector path above
 // spends about 70 G VALU instructions per 16 positions and wave (dot2, DPP row sums, an fma per head and dim; at G = 8
@@ -856,9 +860,9 @@ __device__ __forceinline__ void consume_wave_tile(WaveTile<D>& t, const bf16x8_t
 // MX: the tiles go through the matrix cores (use_mfma). The bound on registers there keeps the accumulators out
 // of AGPRs, which the rescaling would have to move to and fro.
 template <int D, int G, int PPT, int MK, int NT, bool FUSED>
-__global__ void __launch_bounds__(NT, use_mfma(G) ? (D == 128 ? 2 : 3) : 1)
+__global__ void __launch_bounds__(NT, use_mfma(G, MK, FUSED) ? (D == 128 ? 2 : 3) : 1)
     gqa_split_kernel(const int32_t* lens, const int32_t* starts, const int tpr, const Params p) {
-  constexpr bool MX = use_mfma(G);
+  constexpr bool MX = use_mfma(G, MK, FUSED);
   constexpr int NW = NT / kWave;               // waves per workgroup
   constexpr int LPR = D / 8;                   // lanes per KV row, 16 B (8 bf16) each
   constexpr int ROWS = NT / LPR;               // KV rows per load instruction across the workgroup
@@ -1204,11 +1208,11 @@ __global__ void __launch_bounds__(NT, use_mfma(G) ? (D == 128 ? 2 : 3) : 1)
   }
   __syncthreads();
   if (!s_last) return;
-  merge_splits<D, G, NT>(p, z, h, nact, tpr);
+  merge_splits<D, G, NT, MX>(p, z, h, nact, tpr);
 }
 
 // Second-launch merge: one workgroup per (kv head, row).
-template <int D, int G>
+template <int D, int G, bool MX>
 __global__ void __launch_bounds__(kThreads) gqa_combine_kernel(const Params p) {
   const int h = blockIdx.x, z = blockIdx.y;  // z = row * T + token
   int start, end;
@@ -1216,7 +1220,7 @@ __global__ void __launch_bounds__(kThreads) gqa_combine_kernel(const Params p) {
   const int len = end - start;
   const int nact = split_count(len, split_chunk<D>(len, p.splits, p.inv_splits, p.min_chunk));
   if (nact == 1) return;  // the split kernel wrote the output
-  merge_splits<D, G, kThreads>(p, z, h, nact, p.T);
+  merge_splits<D, G, kThreads, MX>(p, z, h, nact, p.T);
 }
 
 // Interval of each additive mask row: first and last position with value > -1e30.
@@ -1326,7 +1330,7 @@ __global__ void __launch_bounds__(kThreads) gqa_probs_kernel(const Params p, flo
 
 template <int D, int G, int MK, int NT, bool FUSED>
 SplitFn pick_ppt(int ppt) {
-  if constexpr (!use_mfma(G))
+  if constexpr (!use_mfma(G, MK, FUSED))
     if (ppt == 2) return gqa_split_kernel<D, G, 2, MK, NT, FUSED>;
   return gqa_split_kernel<D, G, 1, MK, NT, FUSED>;  // the matrix tiles have one form
 }

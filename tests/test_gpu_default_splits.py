@@ -4,7 +4,7 @@ refuses sizes, which does not follow the tuning. The counts are those of a 256-C
 import pytest
 import torch
 
-from breeze_tts_2_flash_amd import default_splits, gqa_decode, workspace_bytes
+from breeze_tts_2_flash_amd import default_splits, gqa_decode, gqa_decode_fused, workspace_bytes
 from tests.test_gpu_parity import assert_close, oracle, rand_case
 from tests.test_zz_no_alloc import BZ_ERR_SCRATCH, noalloc
 
@@ -44,13 +44,36 @@ def test_default_split_count(device, B, NH, NKV, D, cap, splits):
 
 def test_static_scratch_refuses_by_the_largest_default(device):
     """2 rows x 8 kv heads x 8 q heads over 32768 slots: one split per 256 positions is 8.5 MB of partials, refused
-    although the default count is lower and its workspace smaller; an explicit count that fits is taken."""
+    although the default count is lower; an explicit count that fits is taken."""
     q = torch.zeros(2, 64, 128, dtype=torch.bfloat16, device=device)
     kv = torch.zeros(2, 8, 32768, 128, dtype=torch.bfloat16, device=device)
     lens = torch.zeros(2, dtype=torch.int32, device=device)
-    assert workspace_bytes(2, 64, 8, 128, 32768) < 8 << 20
+    assert default_splits(2, 8, 128, 32768) < 128
     rc, _ = noalloc(q, kv, kv, lens, 0.125)
     assert rc == BZ_ERR_SCRATCH
     rc, _ = noalloc(q, kv, kv, lens, 0.125, num_splits=16)
     torch.cuda.synchronize()
     assert rc == 0
+
+
+@pytest.mark.parametrize("B,NKV,G,cap", [(1, 4, 4, 4096), (2, 8, 4, 2048), (4, 8, 2, 3000), (5, 2, 4, 1024), (1, 4, 1, 5000)])
+def test_a_step_keeps_its_bits(device, B, NKV, G, cap):
+    """A fused call with lengths of up to four rows and 4096 positions runs one split per 256 positions or one workgroup
+    per CU, whichever is more (at least 32 positions each); any other takes the tuned count. One workspace of the
+    default size serves both."""
+    from tests.test_gpu_fused import make_step, tens
+
+    cus = torch.cuda.get_device_properties(device).multi_processor_count
+    step = B <= 4 and cap <= 4096
+    old = min(max(-(-cus // (B * NKV)), -(-cap // 256)), -(-cap // 32), 256)
+    splits = old if step else default_splits(B, NKV, 128, cap)
+    assert workspace_bytes(B, NKV * G, NKV, 128, cap) == workspace_bytes(B, NKV * G, NKV, 128, cap, old)
+    s = make_step(cap, B=B, NH=NKV * G, NKV=NKV, cap=cap, pos=cap - 5)
+    lens = torch.full((B,), cap - 4, dtype=torch.int32, device=device)
+    outs = []
+    for n in (0, splits):
+        outs.append(gqa_decode_fused(*(tens(s[k], device) for k in ("qkv", "qn", "kn")), 1e-6, tens(s["cos"], device),
+                                     tens(s["sin"], device), tens(s["kc"], device), tens(s["vc"], device),
+                                     torch.tensor([cap - 5], device=device), 128 ** -0.5, seq_lens=lens, num_splits=n))
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))

@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 import torch
 
-from breeze_tts_2_flash_amd import gqa_decode, gqa_decode_masked
+from breeze_tts_2_flash_amd import gqa_decode, gqa_decode_fused, gqa_decode_masked
 from tests.test_gpu_parity import assert_close, oracle, rand_case
 
 pytestmark = pytest.mark.gpu
@@ -86,9 +86,22 @@ def test_masked_positions_hide_non_finite_values(device, NH, NKV):
 @pytest.mark.parametrize("NH,NKV", GROUPS)
 @pytest.mark.parametrize("pos", [0, 15, 16, 63, 64, 127, 128, 199])
 def test_fused_slot_at_the_edges_of_a_tile(device, NH, NKV, pos):
-    from tests.test_gpu_fused import check_against_oracle, make_step, run_fused
+    from oracle.attention import interval_mask
+    from tests.test_gpu_fused import bits, check_against_oracle, make_step, tens
 
     s = make_step(pos + NH, NH=NH, NKV=NKV, cap=200, pos=pos)
-    for splits in (1, 2):
-        out, kc, vc = run_fused(s, device, pos, [pos + 1, 200], [0, min(pos, 3)], num_splits=splits)
-        check_against_oracle(s, pos, [pos + 1, 200], [0, min(pos, 3)], out, kc, vc, f"pos={pos} splits={splits}")
+    lens, starts = [pos + 1, 200], [0, min(pos, 3)]
+    mask = torch.cat([interval_mask([a], e - 1, 200) for a, e in zip(starts, lens)]).to(device)
+    ranges = [dict(mask=mask)]  # G = 4 with lengths runs on the vector path
+    if NH // NKV == 8:
+        ranges.append(dict(seq_lens=torch.tensor(lens, dtype=torch.int32, device=device),
+                           kv_start=torch.tensor(starts, dtype=torch.int32, device=device)))
+    for kw in ranges:
+        for splits in (1, 2):
+            kc, vc = tens(s["kc"], device), tens(s["vc"], device)
+            out = gqa_decode_fused(tens(s["qkv"], device), tens(s["qn"], device), tens(s["kn"], device), 1e-6,
+                                   tens(s["cos"], device), tens(s["sin"], device), kc, vc,
+                                   torch.tensor([pos], device=device), 128 ** -0.5, num_splits=splits, **kw)
+            torch.cuda.synchronize()
+            check_against_oracle(s, pos, lens, starts, out.float().cpu().numpy(), bits(kc), bits(vc),
+                                 f"pos={pos} splits={splits} {list(kw)}")
