@@ -529,6 +529,186 @@ __global__ void __launch_bounds__(NT)
   p.y[(int64_t)m * p.ldy + n] = f32_to_bf16(v);
 }
 
+// GEMV on the 4x4x4 MFMA (16 blocks). A wave load covers four rows of weights, 256 bytes each: lane 4 b + i holds row i,
+// the 8 k-values 128 c + 8 b .. of chunk c, which are the A operands of two MFMAs (block b: 4 rows x 4 k); lane 4 b + j
+// holds the same 8 k-values of x's row j, their B operands (4 k x up to 4 rows of x). So a block sums its own k-values of
+// all 4 x 4 products into four registers, x costs one 16-byte vector per chunk and lane whatever the number of its rows,
+// its RMSNorm is worked out once per element, and a wave ends with 4 sums per four rows to add over its 16 blocks.
+// Against four dot2 per vector and row of x on the vector unit (the kernels above) that is an eighth of the instructions
+// at four rows of x, where they bound the tail of every workgroup.
+//
+// A workgroup of NW waves owns Q such groups of four rows ("quads"; with the SiLU * up epilogue the first half are gate
+// quads, the second the up quads of the same outputs) and splits k over its waves: wave w takes the TR chunks w, w + NW,
+// ..., so that the workgroup reads NW * 256 consecutive bytes of every row at a time, x once, and every load goes out at
+// once. Each weight segment starts a quad of its own, so a quad has one resource, cut at its last row; lanes past k take
+// an offset outside of it (their loads read 0: a neighbouring row's Inf or NaN must not meet x's padding). The sums meet
+// in LDS.
+template <int Q, int NW, int TR, bool NORM, int EPI>
+__global__ void __launch_bounds__(NW* kWave)
+    gemv_mfma_kernel(const uint16_t* w0, const uint16_t* w1, const uint16_t* w2, int n0, int n1, int ntot, int km,
+                     const uint16_t* x, int64_t ldx, const GemvParams p) {
+  constexpr bool SILU = EPI == BZ_GEMV_SILU_MUL;
+  constexpr int QO = SILU ? Q / 2 : Q;  // quads of outputs
+  constexpr uint32_t kOut = 0x40000000u;  // past every quad (4 k * 2 bytes)
+  const int k = km & 0xffffff, M = km >> 24;  // one preloaded argument
+  const int tid = threadIdx.x, lane = tid % kWave, wave = wave_uniform(tid / kWave);
+  const int j = lane % 4, b = lane / 4;
+
+  // the quads: resource and first output row; segment s has ceil(n_s / 4) of them
+  const int c0 = (n0 + 3) / 4, c1 = (n1 + 3) / 4;
+  auto quad = [&](int qo, bool up, int& row, int& rows) {
+    const int q = blockIdx.x * QO + qo;
+    const uint16_t* base = SILU && up ? w1 : w0;
+    int first = 4 * q, n = n0;
+    row = first;
+    if (!SILU && q >= c0) {
+      const bool third = q >= c0 + c1;
+      base = third ? w2 : w1;
+      first = 4 * (q - c0 - (third ? c1 : 0));
+      n = third ? ntot - n0 - n1 : n1;
+      row = first + n0 + (third ? n1 : 0);
+    }
+    rows = min(4, n - first);  // <= 0 past the last quad: an empty resource
+    return span_rsrc(base + (int64_t)first * k, rows > 0 ? rows * k * 2 : 0);
+  };
+  Rsrc wr[Q];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    int row, rows;
+    wr[q] = quad(SILU ? q % QO : q, SILU && q >= QO, row, rows);
+  }
+  const Rsrc rx = span_rsrc(x, (int)(((int64_t)(M - 1) * ldx + k) * 2));
+  const uint32_t xrow = (uint32_t)(j * ldx) * 2;
+
+  // x first, then every weight load; the prologue waits for x alone
+  uint4 xv[TR], nwv[TR], wt[TR][Q];
+#pragma unroll
+  for (int r = 0; r < TR; ++r) {
+    const int k0 = 128 * (r * NW + wave) + 8 * b;
+    const uint32_t off = k0 < k && j < M ? xrow + 2 * k0 : 0xfffffff0u;
+    xv[r] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rx, off, 0, 0));
+    if (NORM)
+      nwv[r] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(span_rsrc(p.nw, k * 2), 2 * k0, 0, 0));
+  }
+#pragma unroll
+  for (int r = 0; r < TR; ++r) {
+    const int k0 = 128 * (r * NW + wave) + 8 * b;
+    const uint32_t off = k0 < k ? 2 * (j * k + k0) : kOut;
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+      wt[r][q] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(wr[q], off, 0, kStream));
+  }
+  // thread t < 16 Q (the lanes of wave 0 after the sums) writes value v = 4 q + row of row j of x
+  constexpr int NV = 4 * Q;
+  const int v = transposed_index<NV>(tid), vq = v / 4, vr = v % 4;
+  const bool writes = tid < kWave && (Q == 4 || (tid & (Q == 2 ? 4 : 12)) == 0) && vq < QO && j < M;
+  int row = 0, rows = 0;
+  if (tid < kWave) (void)quad(vq, false, row, rows);
+  float resv = 0.f;
+  if (EPI == BZ_GEMV_RESIDUAL) {
+    const Rsrc rr = span_rsrc(p.res, (int)(((int64_t)(M - 1) * p.ldr + ntot) * 2));
+    const uint32_t off = writes && vr < rows ? (uint32_t)((j * p.ldr + row + vr) * 2) : 0xfffffff0u;
+    resv = bf16_to_f32(__builtin_amdgcn_raw_buffer_load_b16(rr, off, 0, 0));
+  }
+  __builtin_amdgcn_sched_barrier(0);
+
+  if (NORM) {
+    __shared__ float s_ss[NW][4];
+    float ss = 0.f;
+#pragma unroll
+    for (int r = 0; r < TR; ++r) {
+      float f[8];
+      unpack8(xv[r], f);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) ss = fmaf(f[i], f[i], ss);
+    }
+    ss += dpp<0x124>(ss);  // row_ror:4 and :8: over the 4 blocks of a 16-lane row (same j)
+    ss += dpp<0x128>(ss);
+    float y = ss;
+    swap16(ss, y);
+    ss += y;
+    y = ss;
+    swap32(ss, y);
+    ss += y;
+    if (lane < 4) s_ss[wave][lane] = ss;
+    __syncthreads();
+    float tot = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) tot += s_ss[w][j];
+    const float rs = rsqrtf(tot * (1.f / (float)k) + p.eps);
+#pragma unroll
+    for (int r = 0; r < TR; ++r) {
+      float f[8], w[8];
+      unpack8(xv[r], f);
+      unpack8(nwv[r], w);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) f[i] *= rs;
+      round8(f);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) f[i] *= w[i];
+      xv[r] = make_uint4(pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3]), pack_bf16x2(f[4], f[5]),
+                         pack_bf16x2(f[6], f[7]));
+    }
+  }
+
+  f32x4_t acc[Q];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) acc[q] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  auto half = [](uint32_t lo, uint32_t hi) { return __builtin_bit_cast(s16x4_t, make_uint2(lo, hi)); };
+#pragma unroll
+  for (int r = 0; r < TR; ++r)
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const uint4 &w = wt[r][q], &u = xv[r];
+      acc[q] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(half(w.x, w.y), half(u.x, u.y), acc[q], 0, 0, 0);
+      acc[q] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(half(w.z, w.w), half(u.z, u.w), acc[q], 0, 0, 0);
+    }
+
+  // the 4 Q sums of a lane over the 16 blocks, transposed over lane bits 5, 4, 3, 2 (transposed_sum's levels; the lanes
+  // of one j stay apart), then over the waves
+  float flat[NV];
+#pragma unroll
+  for (int q = 0; q < Q; ++q)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) flat[4 * q + r] = acc[q][r];
+  swap_level<NV / 2>(flat, true);
+  swap_level<NV / 4>(flat, false);
+  if constexpr (NV >= 8) dpp_level<NV / 8, 0x128>(flat, lane & 8);
+  else flat[0] += dpp<0x128>(flat[0]);
+  auto xor4 = [](float f) {  // lane ^ 4: row_ror:12 for the lanes with bit 2 clear, row_ror:4 for the others
+    const int up = __builtin_amdgcn_update_dpp(0, __float_as_int(f), 0x12c, 0xf, 0xf, true);
+    return __int_as_float(__builtin_amdgcn_update_dpp(up, __float_as_int(f), 0x124, 0xf, 0xa, false));
+  };
+  if constexpr (NV >= 16) {
+    const bool hi = lane & 4;
+    flat[0] = (hi ? flat[1] : flat[0]) + xor4(hi ? flat[0] : flat[1]);
+  } else {
+    flat[0] += xor4(flat[0]);
+  }
+  __shared__ float s_red[NW][kWave];
+  s_red[wave][lane] = flat[0];
+  __syncthreads();
+  if (!writes || vr >= rows) return;
+  float red = 0.f, upv = 0.f;
+  // the lane of the up value: its quad's bit of the value index is lane bit 5
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    red += s_red[w][tid];
+    if (SILU) upv += s_red[w][tid + 32];
+  }
+  float out;
+  if (EPI == BZ_GEMV_PLAIN) {
+    out = red;
+  } else if (EPI == BZ_GEMV_RESIDUAL) {
+    out = resv + bf16_to_f32(f32_to_bf16(red));
+  } else {
+    const float gt = bf16_to_f32(f32_to_bf16(red));
+    const float u = bf16_to_f32(f32_to_bf16(upv));
+    out = bf16_to_f32(f32_to_bf16(gt / (1.f + expf(-gt)))) * u;
+  }
+  p.y[(int64_t)j * p.ldy + row + vr] = f32_to_bf16(out);
+}
+
 // Standalone row RMSNorm, one workgroup per row (bb_fused.cu:219-248).
 __global__ void __launch_bounds__(kGemvThreads) rmsnorm_kernel(const uint16_t* x, int64_t ldx, const uint16_t* w,
                                                                float eps, uint16_t* y, int64_t ldy, int k) {
@@ -678,6 +858,67 @@ GemvFn pick_block(int m, int k, int ntot, int epi, bool norm, int* threads, int*
   return m == 3 ? pick_block_na<3, 512, 2>(na, epi, norm) : pick_block_na<4, 512, 2>(na, epi, norm);
 }
 
+// Where the 4x4x4 MFMA kernel is taken (graph of calls on their own weights, us per call, the other kernels -> this one):
+//   SiLU * up for 2048 < k <= 4096 (x in LDS before), M = 1 / 2 / 4: k 4096, 12288 outputs 41.1 / 42.2 / 47.1 -> 31.8 / 30.8 /
+//     32.9 (6.5 TB/s); 3072, 8192: 19.6 / 20.6 / 23.1 -> 17.8 / 17.7 / 18.2; 2976, 4960: 16.8 / 16.8 / 19.2 -> 12.7 / 12.5 /
+//     13.7; 2560, 6912: 16.1 / 16.2 / 19.0 -> 14.6 / 15.1 / 16.8;
+//   plain there at M >= 3: k 4096, 6144 rows 11.8 / 13.0 -> 11.5 / 12.0 at M = 3 / 4 (M = 1 / 2: 10.7 / 11.1 against 12.4 /
+//     12.6);
+//   at M = 3 also SiLU * up below (k 2048, 6144 outputs 10.6 -> 10.1; 1024, 3072 5.3 -> 4.5; 512, 1536 3.3 -> 3.2), plain past
+//     2048 rows (568, 2560 rows 3.9 -> 3.1) and the residual for 2048 < k <= 4096 (3072, 1024 rows 4.0 -> 3.5). M = 1, 2
+//     and 4 are the rows of a backbone decode step: one stream, a CFG pair, two pairs. There another order of the sums in
+//     one layer travels through the later ones, and the sizes a step has (hidden sizes up to 2048) keep their bits, although
+//     this kernel is faster at M = 4 as well (k 2048, 6144 outputs 11.8 -> 10.3).
+// Up to k = 256 half of its waves would idle.
+bool mfma_route(int m, int k, int rows, int epi) {
+  if (k <= 256 || k > 4096) return false;
+  if (epi == BZ_GEMV_SILU_MUL) return k > 2048 || m == 3;
+  if (epi == BZ_GEMV_PLAIN) return k > 2048 ? m >= 3 : m == 3 && rows > 2048;
+  return k > 2048 && m == 3;
+}
+
+template <int NW, int TR, int Q>
+GemvFn pick_mfma_epi(int epi, bool norm) {
+  if (epi == BZ_GEMV_PLAIN)
+    return norm ? gemv_mfma_kernel<Q, NW, TR, true, BZ_GEMV_PLAIN> : gemv_mfma_kernel<Q, NW, TR, false, BZ_GEMV_PLAIN>;
+  if (epi == BZ_GEMV_RESIDUAL) return norm ? nullptr : gemv_mfma_kernel<Q, NW, TR, false, BZ_GEMV_RESIDUAL>;
+  if constexpr (Q > 1)
+    return norm ? gemv_mfma_kernel<Q, NW, TR, true, BZ_GEMV_SILU_MUL>
+                : gemv_mfma_kernel<Q, NW, TR, false, BZ_GEMV_SILU_MUL>;
+  return nullptr;
+}
+template <int NW, int TR>
+GemvFn pick_mfma_q(int q, int epi, bool norm) {
+  if (q == 4) return pick_mfma_epi<NW, TR, 4>(epi, norm);
+  if (q == 2) return pick_mfma_epi<NW, TR, 2>(epi, norm);
+  return pick_mfma_epi<NW, TR, 1>(epi, norm);
+}
+
+// Four waves up to k = 1024 (one or two chunks each), eight above. Quads per workgroup: the most whose grid fills its
+// last round of CUs to 90% or is long enough (four rounds) for that not to matter; else two, or one where two leave CUs
+// without a workgroup (us per call, 4 / 2 quads: plain at k 4096, 384 / 768 workgroups 12.9 / 12.0; k 2048, 256 / 512: 5.1
+// / 5.7; gate / up at k 2976, 620 / 1240: 13.5 / 12.6; k 2048, 768 / 1536: 10.3 / 11.6; residual at k 3072, 1024 rows: 2
+// quads 3.8, 1 3.3).
+GemvFn pick_mfma(int k, int n0, int n1, int n2, int epi, bool norm, int cus, int* threads, int* grid) {
+  const bool silu = epi == BZ_GEMV_SILU_MUL;
+  const int quads = (n0 + 3) / 4 + (silu ? 0 : (n1 + 3) / 4 + (n2 + 3) / 4);
+  const int nw = k <= 1024 ? 4 : 8;
+  auto groups = [&](int q) { return (quads + (silu ? q / 2 : q) - 1) / (silu ? q / 2 : q); };
+  auto even = [&](int g) { return g >= 4 * cus || 10 * (int64_t)g >= 9 * (int64_t)cus * ((g + cus - 1) / cus); };
+  int q = 4;
+  if (!even(groups(4))) q = silu || groups(2) >= cus ? 2 : 1;
+  *threads = nw * kWave;
+  *grid = groups(q);
+  switch (nw == 4 ? (k <= 512 ? 1 : 2) : 10 * ((k + 1023) / 1024)) {
+    case 1: return pick_mfma_q<4, 1>(q, epi, norm);
+    case 2: return pick_mfma_q<4, 2>(q, epi, norm);
+    case 20: return pick_mfma_q<8, 2>(q, epi, norm);
+    case 30: return pick_mfma_q<8, 3>(q, epi, norm);
+    case 40: return pick_mfma_q<8, 4>(q, epi, norm);
+    default: return nullptr;
+  }
+}
+
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 // Output rows per wave. With x in registers every wave loads its own x, so two rows per wave halve that L2 traffic
@@ -746,6 +987,17 @@ __attribute__((visibility("default"))) int bz_gemv(const bz_gemv_args* a, hipStr
   p.res = static_cast<const uint16_t*>(a->res);
   p.ldr = a->res_stride;
   int bthreads = 0, bgrid = 0;
+  if (mfma_route(a->m, a->k, ntot, a->epilogue)) {
+    int cus = 0;
+    const int rc = bz::device_cu_count(&cus);
+    if (rc != BZ_OK) return rc;
+    GemvFn mf = pick_mfma(a->k, p.n0, p.n1, ntot - p.n0 - p.n1, a->epilogue, a->norm_weight != nullptr, cus, &bthreads,
+                          &bgrid);
+    if (mf == nullptr) return BZ_ERR_UNSUPPORTED;
+    hipLaunchKernelGGL(mf, dim3(bgrid), dim3(bthreads), 0, stream, p.w0, p.w1, p.w2, p.n0, p.n1, p.ntot,
+                       p.k | a->m << 24, p.x, p.ldx, p);
+    return hipGetLastError() == hipSuccess ? BZ_OK : BZ_ERR_LAUNCH;
+  }
   if (GemvFn bf = pick_block(a->m, a->k, ntot, a->epilogue, a->norm_weight != nullptr, &bthreads, &bgrid)) {
     hipLaunchKernelGGL(bf, dim3(bgrid), dim3(bthreads), 0, stream, p.w0, p.w1, p.w2, p.n0, p.n1, p.ntot, p.k, p.x,
                        p.ldx, p);
