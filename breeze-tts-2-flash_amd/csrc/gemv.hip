@@ -864,16 +864,17 @@ GemvFn pick_block(int m, int k, int ntot, int epi, bool norm, int* threads, int*
 //     13.7; 2560, 6912: 16.1 / 16.2 / 19.0 -> 14.6 / 15.1 / 16.8;
 //   plain there at M >= 3: k 4096, 6144 rows 11.8 / 13.0 -> 11.5 / 12.0 at M = 3 / 4 (M = 1 / 2: 10.7 / 11.1 against 12.4 /
 //     12.6);
-//   at M = 3 also SiLU * up below (k 2048, 6144 outputs 10.6 -> 10.1; 1024, 3072 5.3 -> 4.5; 512, 1536 3.3 -> 3.2), plain past
-//     2048 rows (568, 2560 rows 3.9 -> 3.1) and the residual for 2048 < k <= 4096 (3072, 1024 rows 4.0 -> 3.5). M = 1, 2
-//     and 4 are the rows of a backbone decode step: one stream, a CFG pair, two pairs. There another order of the sums in
-//     one layer travels through the later ones, and the sizes a step has (hidden sizes up to 2048) keep their bits, although
+//   at M = 3 also SiLU * up up to k = 1024 (1024, 3072 outputs 5.3 -> 4.5; 512, 1536 3.3 -> 3.2), plain there past 2048
+//     rows (568, 2560 rows 3.9 -> 3.1) and the residual for 2048 < k <= 4096 (3072, 1024 rows 4.0 -> 3.5). M = 1, 2 and 4
+//     are the rows of a backbone decode step: one stream, a CFG pair, two pairs. There another order of the sums in one
+//     layer travels through the later ones, and the sizes a step has (hidden sizes up to 2048) keep their bits, although
 //     this kernel is faster at M = 4 as well (k 2048, 6144 outputs 11.8 -> 10.3).
 // Up to k = 256 half of its waves would idle.
 bool mfma_route(int m, int k, int rows, int epi) {
   if (k <= 256 || k > 4096) return false;
-  if (epi == BZ_GEMV_SILU_MUL) return k > 2048 || m == 3;
-  if (epi == BZ_GEMV_PLAIN) return k > 2048 ? m >= 3 : m == 3 && rows > 2048;
+  const bool three = m == 3 && k <= 1024;
+  if (epi == BZ_GEMV_SILU_MUL) return k > 2048 || three;
+  if (epi == BZ_GEMV_PLAIN) return k > 2048 ? m >= 3 : three && rows > 2048;
   return k > 2048 && m == 3;
 }
 
@@ -909,10 +910,9 @@ GemvFn pick_mfma(int k, int n0, int n1, int n2, int epi, bool norm, int cus, int
   if (!even(groups(4))) q = silu || groups(2) >= cus ? 2 : 1;
   *threads = nw * kWave;
   *grid = groups(q);
-  switch (nw == 4 ? (k <= 512 ? 1 : 2) : 10 * ((k + 1023) / 1024)) {
+  switch (nw == 4 ? (k <= 512 ? 1 : 2) : 10 * ((k + 1023) / 1024)) {  // chunks per wave (mfma_route: no k in 1025..2048)
     case 1: return pick_mfma_q<4, 1>(q, epi, norm);
     case 2: return pick_mfma_q<4, 2>(q, epi, norm);
-    case 20: return pick_mfma_q<8, 2>(q, epi, norm);
     case 30: return pick_mfma_q<8, 3>(q, epi, norm);
     case 40: return pick_mfma_q<8, 4>(q, epi, norm);
     default: return nullptr;
