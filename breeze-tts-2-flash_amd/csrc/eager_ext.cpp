@@ -17,6 +17,7 @@
 #include <hip/hip_runtime_api.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <cmath>
 #include <map>
 #include <string>
 #include <tuple>
@@ -386,6 +387,78 @@ PyObject* fused(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   }
 }
 
+// Devices whose GPU runs the kernels (allow_device; the Python side has asked kernels.device_unsupported).
+constexpr int kMaxDevices = 64;
+bool g_allowed[kMaxDevices];
+
+// hf(query, key, value, mask, scaling) -> out [B, 1, NH, D], or None where the call is not the plain decode call (the
+// conditions of hf_attention._hip_route, a mask of one query row, and a workspace for the stream): the Python path then
+// takes it, with its checks and messages. scaling None: head_dim ** -0.5. One eager transformers call costs mostly host
+// time: 12.3 us a call (B2, 301 of 2048 slots) with the route checks and the output made from Python, 8.3 so.
+PyObject* hf(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (!bound()) return nullptr;
+  if (nargs != 5) {
+    PyErr_SetString(PyExc_TypeError, "hf() takes 5 arguments");
+    return nullptr;
+  }
+  try {
+    for (int i = 0; i < 4; ++i)
+      if (!THPVariable_Check(args[i])) Py_RETURN_NONE;
+    const at::Tensor &q = THPVariable_Unpack(args[0]), &k = THPVariable_Unpack(args[1]), &v = THPVariable_Unpack(args[2]),
+                     &mask = THPVariable_Unpack(args[3]);
+    const at::Device dev = q.device();
+    const auto bf16 = at::kBFloat16;
+    if (q.dim() != 4 || k.dim() != 4 || mask.dim() != 4 || q.size(2) != 1 || !q.is_cuda() || k.device() != dev ||
+        v.device() != dev || mask.device() != dev || dev.index() < 0 || dev.index() >= kMaxDevices ||
+        !g_allowed[dev.index()] || q.scalar_type() != bf16 || k.scalar_type() != bf16 || v.scalar_type() != bf16 ||
+        (mask.scalar_type() != bf16 && mask.scalar_type() != at::kFloat))
+      Py_RETURN_NONE;
+    const int64_t B = q.size(0), NH = q.size(1), D = q.size(3), NKV = k.size(1), cap = k.size(2);
+    const int64_t G = NKV > 0 && NH % NKV == 0 ? NH / NKV : 0;
+    if ((D != 64 && D != 128) || (G != 1 && G != 2 && G != 4 && G != 8) || k.sizes() != v.sizes() ||
+        k.strides() != v.strides() || k.stride(3) != 1 || q.stride(3) != 1 || k.size(0) != B || k.size(3) != D ||
+        mask.size(-1) < cap || mask.stride(-1) != 1 || mask.size(1) != 1 || mask.size(2) != 1 ||
+        (mask.size(0) != B && mask.size(0) != 1))
+      Py_RETURN_NONE;
+    const double scale = args[4] == Py_None ? 1.0 / std::sqrt((double)D) : PyFloat_AsDouble(args[4]);
+    if (PyErr_Occurred()) return nullptr;
+    bz_gqa_decode_args a;
+    std::vector<int64_t> out_shape;
+    fill_args(q, k, v, scale, nullptr, 0, 0, BZ_COMBINE_AUTO, a, out_shape);  // out: [B, NH, D], the same memory
+    mask_view(mask, a.batch, a.capacity, a, dev);
+    const int idx = dev.index();
+    DeviceScope scope(idx);
+    hipStream_t stream = c10::hip::getCurrentHIPStream(idx).stream();
+    const bool noalloc = capturing(stream);
+    const at::Tensor* ws = noalloc ? nullptr : stream_workspace(idx, stream, a);
+    if (!noalloc && ws == nullptr) Py_RETURN_NONE;
+    at::Tensor out = at::empty({B, 1, NH, D}, q.options());
+    a.out = out.data_ptr();
+    if (noalloc) {
+      check_status(g_noalloc(&a, stream), "bz_gqa_decode_noalloc (a call captured without workspace=; pass one for "
+                                          "these sizes)");
+    } else {
+      a.workspace = ws->data_ptr();
+      a.workspace_bytes = (size_t)ws->numel() * ws->element_size();
+      check_status(g_masked(&a, stream), "bz_gqa_decode_masked");
+    }
+    return THPVariable_Wrap(out);
+  } catch (const Error& e) {
+    PyErr_SetString(PyExc_RuntimeError, e.msg.c_str());
+    return nullptr;
+  } catch (const std::exception& e) {
+    PyErr_SetString(PyExc_RuntimeError, e.what());
+    return nullptr;
+  }
+}
+
+PyObject* allow_device(PyObject*, PyObject* arg) {
+  const long idx = PyLong_AsLong(arg);
+  if (PyErr_Occurred()) return nullptr;
+  if (idx >= 0 && idx < kMaxDevices) g_allowed[idx] = true;
+  Py_RETURN_NONE;
+}
+
 // ---- the backbone GEMVs (bz_gemv, bz_rmsnorm)
 
 // x: a bf16 [M, K] device tensor, M 1..4, K and the row stride multiples of 8
@@ -562,6 +635,9 @@ PyMethodDef kMethods[] = {
      "gqa_decode / gqa_decode_masked through the C ABI, or None when the stream has no workspace yet"},
     {"fused", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(fused)), METH_FASTCALL,
      "gqa_decode_fused through the C ABI, or None when the stream has no workspace yet"},
+    {"hf", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(hf)), METH_FASTCALL,
+     "the transformers attention call through the C ABI, or None where the Python path takes it"},
+    {"allow_device", allow_device, METH_O, "a device whose GPU runs the kernels"},
     {"gemv", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(gemv)), METH_FASTCALL,
      "gemv_seg / gemv_resid / gemv_gateup through the C ABI"},
     {"rmsnorm", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(rmsnorm)), METH_FASTCALL,

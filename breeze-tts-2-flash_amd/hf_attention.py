@@ -34,6 +34,7 @@ from .attention import gqa_decode, gqa_decode_masked
 NAME = "mi355_decode"
 EAGER_NAME = "mi355_eager"   # eager_attention alone, for reference runs of a model on the GPU
 calls = {"hip": 0, "eager": 0}
+_native = None   # the native binding's hf(): the route's checks and the call in one, once a call has taken the route
 
 _SUPPORTED_D = (64, 128)
 _SUPPORTED_G = (1, 2, 4, 8)
@@ -100,6 +101,12 @@ def mi355_decode_attention(module, query: torch.Tensor, key: torch.Tensor, value
                            attention_mask: torch.Tensor | None, scaling: float | None = None, dropout: float = 0.0,
                            **kwargs):
     """Attention with the eager signature; q_len == 1 runs the gfx950 split-K kernel (see the module docstring)."""
+    global _native
+    if _native is not None and not (dropout and module.training) and not torch.compiler.is_compiling():
+        out = _native(query, key, value, attention_mask, scaling)
+        if out is not None:
+            calls["hip"] += 1
+            return out, None
     if not _hip_route(module, query, key, value, attention_mask, dropout):
         calls["eager"] += 1
         return _eager(module, query)(module, query, key, value, attention_mask, scaling=scaling, dropout=dropout,
@@ -116,6 +123,10 @@ def mi355_decode_attention(module, query: torch.Tensor, key: torch.Tensor, value
         # the query row's mask ([B, 1, 1, S] at decode already: no slicing view to build)
         mask = attention_mask if attention_mask.size(2) == 1 else attention_mask[:, :, -1:, :]
         gqa_decode_masked(query, key, value, mask, scaling, out)
+    if _native is None and not torch.compiler.is_compiling():
+        eager = kernels.eager()
+        eager.allow_device(query.device.index)
+        _native = eager.hf
     return out, None
 
 
