@@ -19,6 +19,8 @@
 // Where it measured faster (4096 < k <= 6144 at any M, the backbone's down projection; 1024 < k <= 2048 at M >= 3)
 // a block-ordered kernel runs instead: a workgroup streams its rows as one contiguous block, every thread holding one
 // x vector for all of its rows, and the sums are reduced over the workgroup once, at the end (gemv_block_kernel).
+// A third kernel works the products out on the 4x4x4 MFMA, four weight rows per load (gemv_mfma_kernel): for
+// 2048 < k <= 4096 and for M = 3 (mfma_route).
 #include <hip/hip_runtime.h>
 
 #include <math.h>
@@ -380,16 +382,19 @@ __global__ void __launch_bounds__(gemv_threads<KC>())
   }
 }
 
-// Block-ordered GEMV: a workgroup of NT threads owns R = Q * NA output rows (2 R weight rows for the SiLU * up
-// epilogue: the gate rows, then the up rows) and streams them as one contiguous block. A row holds KV = NT / Q vectors
-// of 16 bytes (k <= 8 KV; the vectors past k read 0); load i of thread t reads vector t % KV of row Q i + t / KV, so
-// each wave stays inside one row, every thread needs the same x vector (t % KV) for all of its rows, and all NS loads
-// per thread go out at once. Against the wave-per-row kernel above this keeps the workgroup's bytes in flight
+// Block-ordered GEMV: a workgroup of NT threads owns R output rows (2 R weight rows for the SiLU * up epilogue: the gate
+// rows, then the up rows) and streams them as one contiguous block. Load i of thread t reads the 16 bytes at k = 8 t of
+// row i (k <= 8 NT; past k it reads 0), so every thread needs one x vector per row of x for all of its rows, and all NS
+// loads per thread go out at once. Against the wave-per-row kernel above this keeps the workgroup's bytes in flight
 // contiguous (the wave-per-row kernel with x in LDS holds a third of each of eight rows 12 KB apart at k = 6144) and
 // each workgroup reads x once (with x in registers there every wave reads its own: 32 MB of L2 traffic for q | k | v at
-// M = 4). The sums of a row slot are reduced over the waves of its row group once, at the end: DPP and transposed
-// swaps inside each wave, then the group's waves through LDS in wave order.
-template <int M, int NT, int Q, int NA, bool NORM, int EPI>
+// M = 4). The sums are reduced once, at the end: DPP and transposed swaps inside each wave, then the waves through LDS
+// in wave order. Where a row has no more vectors than a workgroup of 256 threads, four waves finish alone: with 512
+// threads and two rows per load instruction (the same order of sums) a workgroup held 16 rows, its norm, reductions and
+// barriers left eight waves idle together, and two such workgroups fitted on a CU (84 VGPRs) against five of four
+// waves: gate / up at k = 2048, 6144 outputs, M = 3 / 4 11.0 / 11.8 -> 10.4 / 10.3 us (4.9 TB/s), q | k | v 5.0 / 5.4 ->
+// 4.8 / 5.0, o_proj 3.5 -> 3.4.
+template <int M, int NT, int R, bool NORM, int EPI>
 __global__ void __launch_bounds__(NT)
     gemv_block_kernel(const uint16_t* w0, const uint16_t* w1, const uint16_t* w2, int n0, int n1, int ntot, int k,
                       const uint16_t* x, int64_t ldx, const GemvParams args) {
@@ -403,14 +408,10 @@ __global__ void __launch_bounds__(NT)
   p.k = k;
   p.x = x;
   p.ldx = ldx;
-  constexpr int NW = NT / kWave, KV = NT / Q, WPG = NW / Q;  // waves per row group
-  static_assert(KV % kWave == 0, "a wave reads within one row");
+  constexpr int NW = NT / kWave;
   constexpr bool SILU = EPI == BZ_GEMV_SILU_MUL;
-  constexpr int NS = SILU ? 2 * NA : NA;  // weight-row slots per thread (SiLU: the gate slots, then the up slots)
-  constexpr int R = Q * NA;               // output rows per workgroup
+  constexpr int NS = SILU ? 2 * R : R;  // weight-row slots per thread (SiLU: the gate slots, then the up slots)
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
-  const int g = wave_uniform(wave / WPG);  // row group: the weight resources below stay scalar
-  const int kv = tid % KV;
   const int row0 = blockIdx.x * R;
 
   // x (and the norm weight) first, then every weight load; the prologue waits for x alone
@@ -418,16 +419,16 @@ __global__ void __launch_bounds__(NT)
   uint4 xv[M], nwv = make_uint4(0, 0, 0, 0);
 #pragma unroll
   for (int m = 0; m < M; ++m) {
-    const uint32_t off = 8 * kv < p.k ? (uint32_t)(m * p.ldx + 8 * kv) * 2 : 0xfffffff0u;  // past k: reads 0
+    const uint32_t off = 8 * tid < p.k ? (uint32_t)(m * p.ldx + 8 * tid) * 2 : 0xfffffff0u;  // past k: reads 0
     xv[m] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rx, off, 0, 0));
   }
   if (NORM)
-    nwv = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(span_rsrc(p.nw, p.k * 2), 16 * kv, 0, 0));
+    nwv = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(span_rsrc(p.nw, p.k * 2), 16 * tid, 0, 0));
   uint4 wt[NS];
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
-    const bool up = SILU && s >= NA;
-    const int n = row0 + Q * (up ? s - NA : s) + g;
+    const bool up = SILU && s >= R;
+    const int n = row0 + (up ? s - R : s);
     const int bytes = n < p.ntot ? p.k * 2 : 0;  // a row past the last output: an empty resource, its loads read 0
     const uint16_t* base;
     if (SILU) {
@@ -437,7 +438,7 @@ __global__ void __launch_bounds__(NT)
            : n < p.n0 + p.n1 ? p.w1 + (int64_t)(n - p.n0) * p.k
                              : p.w2 + (int64_t)(n - p.n0 - p.n1) * p.k;
     }
-    wt[s] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(span_rsrc(base, bytes), 16 * kv, 0, kStream));
+    wt[s] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(span_rsrc(base, bytes), 16 * tid, 0, kStream));
   }
   // the residual value of the output this thread writes (thread f < R * M: row f / M, batch row f % M); loads past
   // the residual matrix read 0 without a memory access, and values past the output rows are never used
@@ -450,7 +451,6 @@ __global__ void __launch_bounds__(NT)
   __builtin_amdgcn_sched_barrier(0);
 
   if (NORM) {
-    // every row group holds all of x: the sum of squares over the waves of group 0
     __shared__ float s_ss[NW][M];
 #pragma unroll
     for (int m = 0; m < M; ++m) {
@@ -466,7 +466,7 @@ __global__ void __launch_bounds__(NT)
     for (int m = 0; m < M; ++m) {
       float tot = 0.f;
 #pragma unroll
-      for (int w = 0; w < WPG; ++w) tot += s_ss[w][m];
+      for (int w = 0; w < NW; ++w) tot += s_ss[w][m];
       const float rs = rsqrtf(tot * (1.f / (float)p.k) + p.eps);
       float f[8], w[8];
       unpack8(xv[m], f);
@@ -506,15 +506,15 @@ __global__ void __launch_bounds__(NT)
   __shared__ float s_red[NW][NP];
   if (transposed_writer<NP>(lane)) s_red[wave][transposed_index<NP>(lane)] = tot;
   __syncthreads();
-  // thread f < R * M writes row row0 + f / M of batch row f % M: slot a = (f / M) / Q of row group (f / M) % Q
+  // thread f < R * M writes row row0 + f / M of batch row f % M
   if (tid >= R * M) return;
-  const int rr = tid / M, m = tid % M, n = row0 + rr, a = rr / Q, gg = rr % Q;
+  const int r = tid / M, m = tid % M, n = row0 + r;
   if (n >= p.ntot) return;
   float red = 0.f, upv = 0.f;
 #pragma unroll
-  for (int w = 0; w < WPG; ++w) {
-    red += s_red[gg * WPG + w][a * M + m];
-    if (SILU) upv += s_red[gg * WPG + w][(NA + a) * M + m];
+  for (int w = 0; w < NW; ++w) {
+    red += s_red[w][r * M + m];
+    if (SILU) upv += s_red[w][(R + r) * M + m];
   }
   float v;
   if (EPI == BZ_GEMV_PLAIN) {
@@ -799,63 +799,44 @@ GemvFn pick_gemv(int m, int kc, int r, int epi, bool norm, bool pace) {
   }
 }
 
-// The block-ordered kernel where it measured faster than the wave-per-row kernel (cold, graph replay, us per call,
-// wave-per-row -> block):
-//   4096 < k <= 6144, any M: 768 threads, one row per load instruction (down at k = 6144, M = 1 / 2 / 4: 6.71 / 6.77 /
-//     7.50 -> 5.93 / 6.01 / 6.30);
-//   1024 < k <= 2048 and M >= 3: 512 threads, two rows per load instruction (M = 4: q | k | v 7.04 -> 5.41, gate / up
-//     12.75 -> 12.0, o_proj 3.85 -> 3.58). At M <= 2 the wave-per-row kernel with x in registers stays faster there
-//     (the backbone step at M = 2 on one box: gate / up 9.70 against 9.92 us, the step 852 against 861 us).
-// Eight row slots per thread (256 workgroups at the backbone's down and q | k | v), four where eight leave fewer than
-// 256 workgroups (o_proj), and four gate plus four up slots for the SiLU * up epilogue (eight of each: gate / up 11.7
-// against 10.4 us at M = 2).
-constexpr int kBlockMinGrid = 256;
-
-template <int M, int NT, int Q, int NA>
-GemvFn pick_block_epi(int epi, bool norm) {
+// The block-ordered kernel where it measured faster than the wave-per-row kernel (us per call, wave-per-row -> block):
+//   4096 < k <= 6144, any M: 768 threads (down at k = 6144, M = 1 / 2 / 4: 6.71 / 6.77 / 7.50 -> 5.93 / 6.01 / 6.30);
+//   1024 < k <= 2048 and M >= 3: 256 threads (M = 4: q | k | v 7.04 -> 5.0, gate / up 12.75 -> 10.3, o_proj 3.85 -> 3.4).
+//     At M <= 2 the wave-per-row kernel with x in registers stays faster there (the backbone step at M = 2 on one box:
+//     gate / up 9.70 against 9.92 us, the step 852 against 861 us).
+// Eight rows per workgroup (with four, the 256-thread kernel reads x twice as often: q | k | v 5.6 against 5.0, 8000 rows
+// of k = 1056 8.0 against 6.5, o_proj 3.6 against 3.4), four of each kind for the SiLU * up epilogue. There 256 threads
+// take eight gate and eight up rows where that gives every CU two or three workgroups, all that fit at once (133 VGPRs):
+// k 2048, M = 4, four / eight rows: 6144 outputs (768 workgroups of eight) 10.6 / 10.3, k 1536, 4096 (512) 7.0 / 6.6, but
+// k 1280, 2560 (320) 5.6 / 5.9, 1024 (128) 3.7 / 4.2 and k 1888, 7112 (889) 11.3 / 11.4.
+template <int M, int NT, int RS>
+GemvFn pick_block_rows(int epi, bool norm) {
   if (epi == BZ_GEMV_PLAIN)
-    return norm ? gemv_block_kernel<M, NT, Q, NA, true, BZ_GEMV_PLAIN>
-                : gemv_block_kernel<M, NT, Q, NA, false, BZ_GEMV_PLAIN>;
-  if (epi == BZ_GEMV_RESIDUAL) return norm ? nullptr : gemv_block_kernel<M, NT, Q, NA, false, BZ_GEMV_RESIDUAL>;
-  return nullptr;
-}
-template <int M, int NT, int Q>
-GemvFn pick_block_na(int na, int epi, bool norm) {
-  if (epi == BZ_GEMV_SILU_MUL)
-    return norm ? gemv_block_kernel<M, NT, Q, 4, true, BZ_GEMV_SILU_MUL>
-                : gemv_block_kernel<M, NT, Q, 4, false, BZ_GEMV_SILU_MUL>;
-  if constexpr (Q == 1) {
-    (void)na;
-    return pick_block_epi<M, NT, Q, 8>(epi, norm);  // one row per instruction: eight slots
-  } else {
-    return na == 8 ? pick_block_epi<M, NT, Q, 8>(epi, norm) : pick_block_epi<M, NT, Q, 4>(epi, norm);
-  }
+    return norm ? gemv_block_kernel<M, NT, 8, true, BZ_GEMV_PLAIN> : gemv_block_kernel<M, NT, 8, false, BZ_GEMV_PLAIN>;
+  if (epi == BZ_GEMV_RESIDUAL) return norm ? nullptr : gemv_block_kernel<M, NT, 8, false, BZ_GEMV_RESIDUAL>;
+  return norm ? gemv_block_kernel<M, NT, RS, true, BZ_GEMV_SILU_MUL>
+              : gemv_block_kernel<M, NT, RS, false, BZ_GEMV_SILU_MUL>;
 }
 // The block kernel for this call, its workgroup size and grid; nullptr where the wave-per-row kernel is taken.
-GemvFn pick_block(int m, int k, int ntot, int epi, bool norm, int* threads, int* grid) {
-  int q;
+GemvFn pick_block(int m, int k, int ntot, int epi, bool norm, int cus, int* threads, int* grid) {
+  const bool silu = epi == BZ_GEMV_SILU_MUL;
+  auto groups = [&](int rows) { return ntot / rows + (ntot % rows != 0); };
   if (k > 4096 && k <= 6144) {
-    q = 1;
     *threads = 768;
-  } else if (k > 1024 && k <= 2048 && m >= 3) {
-    q = 2;
-    *threads = 512;
-  } else {
-    return nullptr;
-  }
-  int na = 8;
-  if (epi == BZ_GEMV_SILU_MUL || (q == 2 && (ntot + 8 * q - 1) / (8 * q) < kBlockMinGrid)) na = 4;
-  *grid = (ntot + q * na - 1) / (q * na);
-  if (q == 1) {
+    *grid = groups(silu ? 4 : 8);
     switch (m) {
-      case 1: return pick_block_na<1, 768, 1>(na, epi, norm);
-      case 2: return pick_block_na<2, 768, 1>(na, epi, norm);
-      case 3: return pick_block_na<3, 768, 1>(na, epi, norm);
-      case 4: return pick_block_na<4, 768, 1>(na, epi, norm);
-      default: return nullptr;
+      case 1: return pick_block_rows<1, 768, 4>(epi, norm);
+      case 2: return pick_block_rows<2, 768, 4>(epi, norm);
+      case 3: return pick_block_rows<3, 768, 4>(epi, norm);
+      default: return pick_block_rows<4, 768, 4>(epi, norm);
     }
   }
-  return m == 3 ? pick_block_na<3, 512, 2>(na, epi, norm) : pick_block_na<4, 512, 2>(na, epi, norm);
+  if (k <= 1024 || k > 2048 || m < 3) return nullptr;
+  const bool eight = !silu || (groups(8) >= 2 * cus && groups(8) <= 3 * cus);
+  *threads = 256;
+  *grid = groups(eight ? 8 : 4);
+  if (eight) return m == 3 ? pick_block_rows<3, 256, 8>(epi, norm) : pick_block_rows<4, 256, 8>(epi, norm);
+  return m == 3 ? pick_block_rows<3, 256, 4>(epi, norm) : pick_block_rows<4, 256, 4>(epi, norm);
 }
 
 // Where the 4x4x4 MFMA kernel is taken (graph of calls on their own weights, us per call, the other kernels -> this one):
@@ -867,8 +848,8 @@ GemvFn pick_block(int m, int k, int ntot, int epi, bool norm, int* threads, int*
 //   at M = 3 also SiLU * up up to k = 1024 (1024, 3072 outputs 5.3 -> 4.5; 512, 1536 3.3 -> 3.2), plain there past 2048
 //     rows (568, 2560 rows 3.9 -> 3.1) and the residual for 2048 < k <= 4096 (3072, 1024 rows 4.0 -> 3.5). M = 1, 2 and 4
 //     are the rows of a backbone decode step: one stream, a CFG pair, two pairs. There another order of the sums in one
-//     layer travels through the later ones, and the sizes a step has (hidden sizes up to 2048) keep their bits, although
-//     this kernel is faster at M = 4 as well (k 2048, 6144 outputs 11.8 -> 10.3).
+//     layer travels through the later ones, and the sizes a step has (hidden sizes up to 2048) keep their bits: at M = 4 the
+//     block kernel is level there (k 2048, 6144 outputs 10.3 either way).
 // Up to k = 256 half of its waves would idle.
 bool mfma_route(int m, int k, int rows, int epi) {
   if (k <= 256 || k > 4096) return false;
@@ -987,10 +968,10 @@ __attribute__((visibility("default"))) int bz_gemv(const bz_gemv_args* a, hipStr
   p.res = static_cast<const uint16_t*>(a->res);
   p.ldr = a->res_stride;
   int bthreads = 0, bgrid = 0;
+  int cus = 0;
+  const int rc = bz::device_cu_count(&cus);
+  if (rc != BZ_OK) return rc;
   if (mfma_route(a->m, a->k, ntot, a->epilogue)) {
-    int cus = 0;
-    const int rc = bz::device_cu_count(&cus);
-    if (rc != BZ_OK) return rc;
     GemvFn mf = pick_mfma(a->k, p.n0, p.n1, ntot - p.n0 - p.n1, a->epilogue, a->norm_weight != nullptr, cus, &bthreads,
                           &bgrid);
     if (mf == nullptr) return BZ_ERR_UNSUPPORTED;
@@ -998,7 +979,7 @@ __attribute__((visibility("default"))) int bz_gemv(const bz_gemv_args* a, hipStr
                        p.k | a->m << 24, p.x, p.ldx, p);
     return hipGetLastError() == hipSuccess ? BZ_OK : BZ_ERR_LAUNCH;
   }
-  if (GemvFn bf = pick_block(a->m, a->k, ntot, a->epilogue, a->norm_weight != nullptr, &bthreads, &bgrid)) {
+  if (GemvFn bf = pick_block(a->m, a->k, ntot, a->epilogue, a->norm_weight != nullptr, cus, &bthreads, &bgrid)) {
     hipLaunchKernelGGL(bf, dim3(bgrid), dim3(bthreads), 0, stream, p.w0, p.w1, p.w2, p.n0, p.n1, p.ntot, p.k, p.x,
                        p.ldx, p);
     return hipGetLastError() == hipSuccess ? BZ_OK : BZ_ERR_LAUNCH;
@@ -1009,12 +990,7 @@ __attribute__((visibility("default"))) int bz_gemv(const bz_gemv_args* a, hipStr
   const int rows_per_block = threads / kWave * r;
   const int grid = (ntot + rows_per_block - 1) / rows_per_block;
   bool pace = kc > 0 && grid >= kPaceMinGrid;
-  if (pace && (a->epilogue == BZ_GEMV_SILU_MUL ? 2 * r : r) * kc < kPaceMinLoads) {
-    int cus = 0;
-    const int rc = bz::device_cu_count(&cus);
-    if (rc != BZ_OK) return rc;
-    pace = grid > cus;
-  }
+  if (pace && (a->epilogue == BZ_GEMV_SILU_MUL ? 2 * r : r) * kc < kPaceMinLoads) pace = grid > cus;
   GemvFn fn = pick_gemv(a->m, kc, r, a->epilogue, a->norm_weight != nullptr, pace);
   if (fn == nullptr) return BZ_ERR_UNSUPPORTED;
   hipLaunchKernelGGL(fn, dim3(grid), dim3(threads), kc > 0 ? 0 : lds, stream, p.w0, p.w1, p.w2, p.n0, p.n1, p.ntot,
