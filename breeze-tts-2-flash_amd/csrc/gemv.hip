@@ -804,39 +804,56 @@ GemvFn pick_gemv(int m, int kc, int r, int epi, bool norm, bool pace) {
 //   1024 < k <= 2048 and M >= 3: 256 threads (M = 4: q | k | v 7.04 -> 5.0, gate / up 12.75 -> 10.3, o_proj 3.85 -> 3.4).
 //     At M <= 2 the wave-per-row kernel with x in registers stays faster there (the backbone step at M = 2 on one box:
 //     gate / up 9.70 against 9.92 us, the step 852 against 861 us).
-// Eight rows per workgroup (with four, the 256-thread kernel reads x twice as often: q | k | v 5.6 against 5.0, 8000 rows
-// of k = 1056 8.0 against 6.5, o_proj 3.6 against 3.4), four of each kind for the SiLU * up epilogue. There 256 threads
-// take eight gate and eight up rows where that gives every CU two or three workgroups, all that fit at once (133 VGPRs):
-// k 2048, M = 4, four / eight rows: 6144 outputs (768 workgroups of eight) 10.6 / 10.3, k 1536, 4096 (512) 7.0 / 6.6, but
-// k 1280, 2560 (320) 5.6 / 5.9, 1024 (128) 3.7 / 4.2 and k 1888, 7112 (889) 11.3 / 11.4.
-template <int M, int NT, int RS>
+// Eight rows per workgroup: with four, x is read twice as often (256 threads: q | k | v 5.6 against 5.0, 8000 rows of
+// k = 1056 8.0 against 6.5, o_proj 3.6 against 3.4; 768 threads, k 6144, M = 4: 2048 rows 6.3 against 6.15, 4096 rows 10.3
+// against 9.7). Four of them with 768 threads where eight leave half of the CUs without a workgroup, or a second round
+// at most half full (M = 1 / 2 / 4, eight -> four: k 6144, 1024 rows 4.50 / 4.43 / 4.88 -> 3.96 / 4.06 / 4.25; 2560 rows
+// 7.71 / 7.84 / 8.45 -> 7.03 / 7.08 / 7.90; k 4960, 2976 rows 7.30 / 7.20 / 7.85 -> 6.65 / 6.71 / 7.49; k 5120, 1536 rows,
+// 192 workgroups of eight: 4.67 / 4.56 / 4.95 against 4.71 / 4.87 / 5.37; two rows: 8.9 at k 6144, 2560 rows, M = 4).
+// Four of each kind for the SiLU * up epilogue. There 256 threads take eight gate and eight up rows where that gives
+// every CU two or three workgroups, all that fit at once (133 VGPRs): k 2048, M = 4, four / eight rows: 6144 outputs (768
+// workgroups of eight) 10.6 / 10.3, k 1536, 4096 (512) 7.0 / 6.6, but k 1280, 2560 (320) 5.6 / 5.9, 1024 (128) 3.7 / 4.2 and
+// k 1888, 7112 (889) 11.3 / 11.4.
+template <int M, int NT, int R>
 GemvFn pick_block_rows(int epi, bool norm) {
-  if (epi == BZ_GEMV_PLAIN)
-    return norm ? gemv_block_kernel<M, NT, 8, true, BZ_GEMV_PLAIN> : gemv_block_kernel<M, NT, 8, false, BZ_GEMV_PLAIN>;
-  if (epi == BZ_GEMV_RESIDUAL) return norm ? nullptr : gemv_block_kernel<M, NT, 8, false, BZ_GEMV_RESIDUAL>;
-  return norm ? gemv_block_kernel<M, NT, RS, true, BZ_GEMV_SILU_MUL>
-              : gemv_block_kernel<M, NT, RS, false, BZ_GEMV_SILU_MUL>;
+  if (epi == BZ_GEMV_SILU_MUL) {
+    if constexpr (R == 4 || NT == 256)
+      return norm ? gemv_block_kernel<M, NT, R, true, BZ_GEMV_SILU_MUL>
+                  : gemv_block_kernel<M, NT, R, false, BZ_GEMV_SILU_MUL>;
+    return nullptr;
+  }
+  if constexpr (R == 8 || NT == 768) {
+    if (epi == BZ_GEMV_PLAIN)
+      return norm ? gemv_block_kernel<M, NT, R, true, BZ_GEMV_PLAIN> : gemv_block_kernel<M, NT, R, false, BZ_GEMV_PLAIN>;
+    return norm ? nullptr : gemv_block_kernel<M, NT, R, false, BZ_GEMV_RESIDUAL>;
+  }
+  return nullptr;
+}
+template <int M, int NT>
+GemvFn pick_block_m(bool eight, int epi, bool norm) {
+  return eight ? pick_block_rows<M, NT, 8>(epi, norm) : pick_block_rows<M, NT, 4>(epi, norm);
 }
 // The block kernel for this call, its workgroup size and grid; nullptr where the wave-per-row kernel is taken.
 GemvFn pick_block(int m, int k, int ntot, int epi, bool norm, int cus, int* threads, int* grid) {
   const bool silu = epi == BZ_GEMV_SILU_MUL;
   auto groups = [&](int rows) { return ntot / rows + (ntot % rows != 0); };
+  const int g8 = groups(8);
   if (k > 4096 && k <= 6144) {
+    const bool eight = !silu && (g8 > cus / 2 && (g8 <= cus || g8 > cus + cus / 2));
     *threads = 768;
-    *grid = groups(silu ? 4 : 8);
+    *grid = eight ? g8 : groups(4);
     switch (m) {
-      case 1: return pick_block_rows<1, 768, 4>(epi, norm);
-      case 2: return pick_block_rows<2, 768, 4>(epi, norm);
-      case 3: return pick_block_rows<3, 768, 4>(epi, norm);
-      default: return pick_block_rows<4, 768, 4>(epi, norm);
+      case 1: return pick_block_m<1, 768>(eight, epi, norm);
+      case 2: return pick_block_m<2, 768>(eight, epi, norm);
+      case 3: return pick_block_m<3, 768>(eight, epi, norm);
+      default: return pick_block_m<4, 768>(eight, epi, norm);
     }
   }
   if (k <= 1024 || k > 2048 || m < 3) return nullptr;
-  const bool eight = !silu || (groups(8) >= 2 * cus && groups(8) <= 3 * cus);
+  const bool eight = !silu || (g8 >= 2 * cus && g8 <= 3 * cus);
   *threads = 256;
-  *grid = groups(eight ? 8 : 4);
-  if (eight) return m == 3 ? pick_block_rows<3, 256, 8>(epi, norm) : pick_block_rows<4, 256, 8>(epi, norm);
-  return m == 3 ? pick_block_rows<3, 256, 4>(epi, norm) : pick_block_rows<4, 256, 4>(epi, norm);
+  *grid = eight ? g8 : groups(4);
+  return m == 3 ? pick_block_m<3, 256>(eight, epi, norm) : pick_block_m<4, 256>(eight, epi, norm);
 }
 
 // Where the 4x4x4 MFMA kernel is taken (graph of calls on their own weights, us per call, the other kernels -> this one):

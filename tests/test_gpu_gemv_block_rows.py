@@ -1,6 +1,6 @@
-"""The block-ordered GEMV with 256 threads (1024 < k <= 2048, three or four rows of x) where it can go wrong: k on each
-side of its range, k that leaves lanes idle, both row counts per workgroup with a ragged last workgroup, segments that
-end inside a workgroup. Against the GEMV oracle, with its tolerance."""
+"""The block-ordered GEMV (256 threads for 1024 < k <= 2048 and three or four rows of x, 768 for 4096 < k <= 6144) where it
+can go wrong: k on each side of its ranges, k that leaves lanes idle, both row counts per workgroup with a ragged last
+workgroup, segments that end inside a workgroup. Against the GEMV oracle, with its tolerance."""
 import numpy as np
 import pytest
 import torch
@@ -37,6 +37,17 @@ def test_segments_and_residual(device, M, K, ns):
     torch.cuda.synchronize()
     assert_gemv_close(host_bits(y), gemv_ref(x, [w for w in W if w.shape[0]], nw, 1e-6), f"seg M={M} K={K} ns={ns}")
     w = np.concatenate(W)
+    gemv_resid(dev(x, device), dev(w, device), dev(res, device), y)
+    torch.cuda.synchronize()
+    assert_gemv_close(host_bits(y), gemv_ref(x, [w], epilogue="residual", res_bits=res), f"resid M={M} K={K} N={N}")
+
+
+@pytest.mark.parametrize("M", [1, 2, 4])
+@pytest.mark.parametrize("K,N", [(4104, 1), (6144, 1022), (4960, 1027), (4104, 2051), (5000, 3073)])
+def test_long_rows(device, M, K, N):
+    rng = np.random.default_rng(M * K + N)
+    x, w, res = rand_bits(rng, M, K), rand_bits(rng, N, K, scale=K ** -0.5), rand_bits(rng, M, N)
+    y = torch.empty(M, N, dtype=torch.bfloat16, device=device)
     gemv_resid(dev(x, device), dev(w, device), dev(res, device), y)
     torch.cuda.synchronize()
     assert_gemv_close(host_bits(y), gemv_ref(x, [w], epilogue="residual", res_bits=res), f"resid M={M} K={K} N={N}")
