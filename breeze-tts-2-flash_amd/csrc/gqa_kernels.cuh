@@ -420,8 +420,8 @@ __device__ __forceinline__ bool any_valid(const uint32_t* bits, int shift, int l
 
 // One wave's part of a mask scan: `keep` bit i of lane l stands for position first + VPL * l + i (VPL consecutive
 // positions per lane). lo and hi, uniform over the wave, take in the first and last kept position (ballots and scalar
-// bit counts; a butterfly of min / max over the lanes took twelve LDS permutes), and the 64-position blocks that hold
-// one are recorded in bits (blocks of 1 << shift positions).
+// bit counts; a butterfly of min / max over the lanes took twelve LDS permutes), and the blocks of 1 << shift positions
+// that hold one are recorded in bits, from each run of 64 positions (shift >= 6: a run lies in one block).
 template <int VPL>
 __device__ __forceinline__ void mask_note(uint32_t keep, int first, int lane, int shift, int& lo, int& hi,
                                           uint32_t* bits) {
@@ -433,7 +433,7 @@ __device__ __forceinline__ void mask_note(uint32_t keep, int first, int lane, in
   lo = min(lo, first + VPL * f + __builtin_ctz(kf));
   hi = max(hi, first + VPL * t + 31 - __builtin_clz(kt));
   if (bits == nullptr) return;
-  constexpr int LPB = 64 / VPL;  // lanes per block of 64 positions; first is a multiple of 64 * VPL
+  constexpr int LPB = 64 / VPL;  // lanes per run of 64 positions; first is a multiple of 64 * VPL
   if (lane < VPL && ((any >> (LPB * lane % 64)) & (LPB == 64 ? ~0ull : (1ull << (LPB % 64)) - 1)) != 0) {
     const int blk = (first + 64 * lane) >> shift;
     atomicOr(&bits[blk >> 5], 1u << (blk & 31));
@@ -449,7 +449,8 @@ __device__ __forceinline__ void mask_note(uint32_t keep, int first, int lane, in
 // aligned is read 16 bytes per lane (one load per thread covers 2048 bf16 positions), its last cap % VPL positions and
 // any other row value by value, 8 loads per thread in flight. The row goes through a buffer resource cut at cap: every
 // load is unconditional, and loads past it read 0 and touch no memory. Fused step, B2, 1377 of 2048 slots, bf16 mask, us
-// per call: 8.68 with 2-byte loads and lane butterflies, 8.15 so (6.5 with the range from seq_lens at 1024).
+// per call: 8.68 with 2-byte loads and lane butterflies, 8.15 so (6.5 with the range from seq_lens at 1024). Plain call, 2
+// rows of 140000 slots (blocks of 128 positions), bf16 / fp32 mask: 132.9 / 123.9 value by value, 70.8 / 72.1 so.
 template <int NT, int MK>
 __device__ void mask_row_range_t(const void* row, int cap, int& start, int& end, uint32_t* bits) {
   constexpr int kBytes = MK == BZ_MASK_BF16 ? 2 : 4, VPL = 16 / kBytes;
@@ -467,7 +468,7 @@ __device__ void mask_row_range_t(const void* row, int cap, int& start, int& end,
     __syncthreads();
   };
   int lo = cap, hi = -1;
-  // kU batches of one position per lane, NT positions apart, from base; positions past cap (or below from) do not count
+  // kU batches of one position per lane, NT positions apart, from base; positions past cap do not count
   auto singles = [&](auto ku, int base, bool first) {
     constexpr int kU = decltype(ku)::value;
     float m[kU];
@@ -505,7 +506,7 @@ __device__ void mask_row_range_t(const void* row, int cap, int& start, int& end,
       mask_note<VPL>(keep, base + (u * NT + wave * kWave) * VPL, lane, shift, lo, hi, bits);
     }
   };
-  if ((reinterpret_cast<uintptr_t>(row) & 15) == 0 && (bits == nullptr || shift == 6)) {
+  if ((reinterpret_cast<uintptr_t>(row) & 15) == 0) {
     const int whole = cap / VPL * VPL;
     const int pos = whole + lane;  // the last cap % VPL positions: a lane each, by every wave
     const float rest = value(pos);
@@ -519,7 +520,8 @@ __device__ void mask_row_range_t(const void* row, int cap, int& start, int& end,
     if (last != 0) {
       lo = min(lo, whole + __builtin_ctzll(last));
       hi = max(hi, whole + 63 - __builtin_clzll(last));
-      if (bits != nullptr && tid == 0) atomicOr(&bits[whole >> 11], 1u << ((whole >> 6) & 31));
+      // cap - whole < VPL: one block
+      if (bits != nullptr && tid == 0) atomicOr(&bits[whole >> (shift + 5)], 1u << ((whole >> shift) & 31));
     }
   } else {
     for (int base = 0; base < cap; base += 8 * NT) singles(std::integral_constant<int, 8>{}, base, base == 0);

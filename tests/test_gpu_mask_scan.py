@@ -42,7 +42,7 @@ def test_single_positions_and_intervals(device, dtype, aligned, cap):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("aligned", [True, False])
-@pytest.mark.parametrize("cap", [70, 2047, 2304, 8199])
+@pytest.mark.parametrize("cap", [70, 2047, 2304, 8199, 131073, 140005, 270001])  # blocks of 64, 128 and 256 positions
 def test_chunks_are_skipped_or_kept(device, dtype, aligned, cap):
     """Attended positions are few and far apart, so most chunks are skipped; a position whose block went unrecorded would
     be missing from the result."""
