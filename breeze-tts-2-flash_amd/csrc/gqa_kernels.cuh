@@ -421,10 +421,11 @@ __device__ __forceinline__ bool any_valid(const uint32_t* bits, int shift, int l
 // One wave's part of a mask scan: `keep` bit i of lane l stands for position first + VPL * l + i (VPL consecutive
 // positions per lane). lo and hi, uniform over the wave, take in the first and last kept position (ballots and scalar
 // bit counts; a butterfly of min / max over the lanes took twelve LDS permutes), and the blocks of 1 << shift positions
-// that hold one are recorded in bits, from each run of 64 positions (shift >= 6: a run lies in one block).
+// that hold one are recorded in bits, from each run of 64 positions (shift >= 6). Runs that start inside a block (inside)
+// count for both blocks they touch, which at most streams a chunk that could have been skipped.
 template <int VPL>
-__device__ __forceinline__ void mask_note(uint32_t keep, int first, int lane, int shift, int& lo, int& hi,
-                                          uint32_t* bits) {
+__device__ __forceinline__ void mask_note(uint32_t keep, int first, int cap, int lane, int shift, bool inside, int& lo,
+                                          int& hi, uint32_t* bits) {
   const uint64_t any = __ballot(keep != 0);
   if (any == 0) return;
   const int f = __builtin_ctzll(any), t = 63 - __builtin_clzll(any);
@@ -433,10 +434,14 @@ __device__ __forceinline__ void mask_note(uint32_t keep, int first, int lane, in
   lo = min(lo, first + VPL * f + __builtin_ctz(kf));
   hi = max(hi, first + VPL * t + 31 - __builtin_clz(kt));
   if (bits == nullptr) return;
-  constexpr int LPB = 64 / VPL;  // lanes per run of 64 positions; first is a multiple of 64 * VPL
-  if (lane < VPL && ((any >> (LPB * lane % 64)) & (LPB == 64 ? ~0ull : (1ull << (LPB % 64)) - 1)) != 0) {
+  constexpr int LPB = 64 / VPL;  // lanes per run of 64 positions
+  if (lane < VPL && ((any >> (LPB * lane)) & ((1ull << LPB) - 1)) != 0) {
     const int blk = (first + 64 * lane) >> shift;
     atomicOr(&bits[blk >> 5], 1u << (blk & 31));
+    if (inside) {
+      const int last = min(first + 64 * lane + 63, cap - 1) >> shift;
+      atomicOr(&bits[last >> 5], 1u << (last & 31));
+    }
   }
 }
 
@@ -445,12 +450,13 @@ __device__ __forceinline__ void mask_note(uint32_t keep, int first, int lane, in
 // (kValidWords words of LDS), the blocks holding attended positions are recorded there too (valid_shift(cap)), so a
 // workgroup can skip a chunk the mask excludes entirely, as the reference skips its fully masked 64-position chunks
 // (bb_attn.cu:9-11, :151-154).
-// The scan stands before a workgroup's first K/V load, so it is bound by its round trip. A row whose start is 16-byte
-// aligned is read 16 bytes per lane (one load per thread covers 2048 bf16 positions), its last cap % VPL positions and
-// any other row value by value, 8 loads per thread in flight. The row goes through a buffer resource cut at cap: every
-// load is unconditional, and loads past it read 0 and touch no memory. Fused step, B2, 1377 of 2048 slots, bf16 mask, us
-// per call: 8.68 with 2-byte loads and lane butterflies, 8.15 so (6.5 with the range from seq_lens at 1024). Plain call, 2
-// rows of 140000 slots (blocks of 128 positions), bf16 / fp32 mask: 132.9 / 123.9 value by value, 70.8 / 72.1 so.
+// The scan stands before a workgroup's first K/V load, so it is bound by its round trip. The row is read 16 bytes per
+// lane from its first 16-byte boundary on (one load per thread covers 2048 bf16 positions); the positions before it and
+// the rest at the end, fewer than VPL each, take one load of a position per lane. The row goes through a buffer resource
+// cut at cap: every load is unconditional, and loads past it read 0 and touch no memory. us per call, value by value / so:
+// fused step, B2, 1377 of 2048 slots, bf16 mask 8.68 / 8.15 (6.5 with the range from seq_lens at 1024); plain call, 2 rows of
+// 140000 slots (blocks of 128 positions), bf16 mask 132.9 / 70.8, fp32 123.9 / 72.1; rows that start 2 bytes past a boundary,
+// bf16, 2 rows x 8 kv heads x 4096 13.8 / 12.6, 2 x 1 x 20000 23.2 / 15.1.
 template <int NT, int MK>
 __device__ void mask_row_range_t(const void* row, int cap, int& start, int& end, uint32_t* bits) {
   constexpr int kBytes = MK == BZ_MASK_BF16 ? 2 : 4, VPL = 16 / kBytes;
@@ -458,38 +464,26 @@ __device__ void mask_row_range_t(const void* row, int cap, int& start, int& end,
   const int tid = threadIdx.x, lane = tid % kWave, wave = wave_uniform(tid / kWave);
   const int shift = valid_shift(cap);
   const Rsrc rm = span_rsrc(row, cap * kBytes);
-  auto value = [&](int pos) {
-    return MK == BZ_MASK_BF16 ? bf16_to_f32(__builtin_amdgcn_raw_buffer_load_b16(rm, (uint32_t)pos * kBytes, 0, 0))
-                              : __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rm, (uint32_t)pos * kBytes, 0, 0));
-  };
-  auto clear = [&] {  // after the first loads are issued
-    if (bits == nullptr) return;
-    for (int i = tid; i < kValidWords; i += NT) bits[i] = 0;
-    __syncthreads();
-  };
+  const int head = min(cap, (int)(-reinterpret_cast<uintptr_t>(row) & 15) / kBytes);  // positions before the boundary
+  const int whole = (cap - head) / VPL * VPL, tail = head + whole;
+  auto ends_pos = [&](int l) { return l < head ? l : tail + l - head; };  // the head's and the tail's, a lane each
+  const int epos = ends_pos(lane);
+  const uint32_t eoff = (uint32_t)epos * kBytes;
+  const float ends = MK == BZ_MASK_BF16 ? bf16_to_f32(__builtin_amdgcn_raw_buffer_load_b16(rm, eoff, 0, 0))
+                                        : __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rm, eoff, 0, 0));
   int lo = cap, hi = -1;
-  // kU batches of one position per lane, NT positions apart, from base; positions past cap do not count
-  auto singles = [&](auto ku, int base, bool first) {
-    constexpr int kU = decltype(ku)::value;
-    float m[kU];
-#pragma unroll
-    for (int u = 0; u < kU; ++u) m[u] = value(base + u * NT + tid);
-    if (first) clear();
-#pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      const int pos = base + u * NT + tid;
-      mask_note<1>(pos < cap && m[u] > kExcluded, base + u * NT + wave * kWave, lane, shift, lo, hi, bits);
-    }
-  };
-  // the same for kU loads of VPL positions per lane
-  auto vectors = [&](auto ku, int base, int whole, bool first) {
+  // kU loads of VPL positions per lane, from position head + base
+  auto vectors = [&](auto ku, int base) {
     constexpr int kU = decltype(ku)::value;
     uint4 w[kU];
 #pragma unroll
     for (int u = 0; u < kU; ++u)
-      w[u] = __builtin_bit_cast(
-          uint4, __builtin_amdgcn_raw_buffer_load_b128(rm, (uint32_t)(base + (u * NT + tid) * VPL) * kBytes, 0, 0));
-    if (first) clear();
+      w[u] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
+                                           rm, (uint32_t)(head + base + (u * NT + tid) * VPL) * kBytes, 0, 0));
+    if (base == 0 && bits != nullptr) {  // after the first loads are issued
+      for (int i = tid; i < kValidWords; i += NT) bits[i] = 0;
+      __syncthreads();
+    }
 #pragma unroll
     for (int u = 0; u < kU; ++u) {
       float f[8];
@@ -503,28 +497,26 @@ __device__ void mask_row_range_t(const void* row, int cap, int& start, int& end,
 #pragma unroll
       for (int i = 0; i < VPL; ++i) keep |= f[i] > kExcluded ? 1u << i : 0u;
       if (base + (u * NT + tid) * VPL >= whole) keep = 0;
-      mask_note<VPL>(keep, base + (u * NT + wave * kWave) * VPL, lane, shift, lo, hi, bits);
+      mask_note<VPL>(keep, head + base + (u * NT + wave * kWave) * VPL, cap, lane, shift, head != 0, lo,
+                     hi, bits);
     }
   };
-  if ((reinterpret_cast<uintptr_t>(row) & 15) == 0) {
-    const int whole = cap / VPL * VPL;
-    const int pos = whole + lane;  // the last cap % VPL positions: a lane each, by every wave
-    const float rest = value(pos);
-    if (cap <= NT * VPL) {
-      vectors(std::integral_constant<int, 1>{}, 0, whole, true);
-    } else {
-      for (int base = 0; base < whole; base += 4 * NT * VPL)
-        vectors(std::integral_constant<int, 4>{}, base, whole, base == 0);
-    }
-    const uint64_t last = __ballot(pos < cap && rest > kExcluded);
-    if (last != 0) {
-      lo = min(lo, whole + __builtin_ctzll(last));
-      hi = max(hi, whole + 63 - __builtin_clzll(last));
-      // cap - whole < VPL: one block
-      if (bits != nullptr && tid == 0) atomicOr(&bits[whole >> (shift + 5)], 1u << ((whole >> shift) & 31));
-    }
+  if (whole <= NT * VPL) {
+    vectors(std::integral_constant<int, 1>{}, 0);
   } else {
-    for (int base = 0; base < cap; base += 8 * NT) singles(std::integral_constant<int, 8>{}, base, base == 0);
+    for (int base = 0; base < whole; base += 4 * NT * VPL) vectors(std::integral_constant<int, 4>{}, base);
+  }
+  const uint64_t any = __ballot(epos < cap && ends > kExcluded);
+  if (any != 0) {
+    lo = min(lo, ends_pos(__builtin_ctzll(any)));
+    hi = max(hi, ends_pos(63 - __builtin_clzll(any)));
+    if (bits != nullptr && tid == 0) {
+      if (any & ((1ull << head) - 1)) atomicOr(&bits[0], 1u);
+      if (any >> head) {  // cap - tail < VPL: one block, or the two that meet there
+        atomicOr(&bits[tail >> (shift + 5)], 1u << ((tail >> shift) & 31));
+        if (head != 0) atomicOr(&bits[(cap - 1) >> (shift + 5)], 1u << (((cap - 1) >> shift) & 31));
+      }
+    }
   }
   if (lane == 0) {
     s_lo[wave] = lo;

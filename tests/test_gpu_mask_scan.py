@@ -1,6 +1,7 @@
-"""The mask scan (mask_interval, and the range and chunk skipping of the masked attention) on each of its paths: rows that
-start 16-byte aligned (16-byte loads, the last few positions apart) and rows that do not, capacities around the sizes of
-a lane's load, a wave's and a workgroup's, single kept positions at their edges, both mask types."""
+"""The mask scan (mask_interval, and the range and chunk skipping of the masked attention): rows that start 16-byte aligned
+and rows that start anywhere before a 16-byte boundary (the positions before it and the last few take loads of their own),
+capacities around the sizes of a lane's load, a wave's and a workgroup's and of the skip map's blocks, single kept
+positions at their edges, both mask types."""
 import numpy as np
 import pytest
 import torch
@@ -61,3 +62,32 @@ def test_chunks_are_skipped_or_kept(device, dtype, aligned, cap):
         out = gqa_decode_masked(q.to(device), k.to(device), v.to(device), mask, D ** -0.5, num_splits=splits)
         got = out.float().cpu().numpy()
         assert (np.abs(got - ref) <= 2e-3 + 1e-2 * np.abs(ref)).all(), (cap, splits)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("cap", [1, 3, 6, 8, 13, 71, 2055, 131080])
+def test_every_row_start(device, dtype, cap):
+    """Rows that start 0 .. 7 elements past a 16-byte boundary: one kept position at either end, at the first boundary and
+    around the first two blocks' edges, alone in its row (interval), and all of them together (chunk skipping)."""
+    esize = torch.tensor([], dtype=dtype).element_size()
+    for off in range(16 // esize):
+        head = -off % (16 // esize)
+        at = sorted({p for p in (0, head - 1, head, head + 63, head + 64, 63, 64, 127, 128, cap - 2, cap - 1) if 0 <= p < cap})
+        pitch = (cap + 31) // 16 * 16
+        rows = torch.full((len(at) + 1, pitch), NEG, dtype=dtype, device=device)
+        m = rows[:, off:off + cap]
+        for i, p in enumerate(at):
+            m[i, p] = m[-1, p] = 0.5
+        lens, starts = mask_interval(m, cap)
+        torch.cuda.synchronize()
+        want = [(p, p + 1) for p in at] + [(at[0], at[-1] + 1)]
+        assert [tuple(r) for r in zip(starts.tolist(), lens.tolist())] == want, off
+        if cap > 2055:
+            continue
+        g = torch.Generator().manual_seed(off)
+        q, k, v = (torch.randn(s, generator=g).bfloat16() for s in ((1, 4, 64), (1, 2, cap, 64), (1, 2, cap, 64)))
+        ref = decode_attention(q.float().numpy(), k.float().numpy(), v.float().numpy(), np.full(1, cap), 0.125,
+                               mask=m[-1:].float().cpu().numpy())
+        for splits in (0, 9):
+            out = gqa_decode_masked(q.to(device), k.to(device), v.to(device), m[-1:], 0.125, num_splits=splits)
+            assert (np.abs(out.float().cpu().numpy() - ref) <= 2e-3 + 1e-2 * np.abs(ref)).all(), (off, splits)
