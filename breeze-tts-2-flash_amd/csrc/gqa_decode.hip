@@ -130,12 +130,18 @@ int most_splits_for(int64_t units, int D, int len, int cus) {
 //     splits 23.8, 8 25.7, 16 26.3).
 //   - Past kMergeBatch splits the merge takes a second batch of partials: worth it up to two batches for chunks of 32 KB
 //     of K+V (1 row of 2048: 16 splits 6.61, 32 6.28; of 4096: 8.24, 7.50; 2 kv heads, G 4, 1000 positions: 16 splits
-//     5.43, 32 6.03), and beyond for chunks of 128 KB (1 kv head x 8192: 16 splits 10.7, 32 8.0, 256 13.7).
+//     5.43, 32 6.03), and beyond for chunks of 128 KB (1 kv head x 8192: 16 splits 10.7, 32 8.0, 256 13.7). Never a little
+//     more than those 32 KB, one tile pair: a chunk of 66 positions takes a third tile (1 row of 1500: 23 splits 6.48, 24
+//     6.14; 2 kv heads, G 4: 6.67, 6.22; 1 row x 1 kv head 5.97, 5.63).
 //   - Rows of up to twice kOneSplitBytes are not split where the rows alone take half of the CUs (16 rows of 200: 1 split
 //     6.09, 2 7.00; 8 such rows: 5.72, 6.39).
 int default_splits_for(int rows, int NKV, int D, int len, int cus) {
   constexpr int kMergeBatch = 16, kPairRows = 3;
-  const int64_t units = (int64_t)rows * NKV, kb = (int64_t)len * D / 256;
+  const int64_t units = (int64_t)rows * NKV;
+  auto raised = [&](int s, int kb) {  // to chunks of kb KB of K+V, rounded up, where more than s whole ones fit
+    const int64_t n = (int64_t)len * D, per = 256 * kb;
+    return n / per > s ? (int)((n + per - 1) / per) : s;
+  };
   if (2 * units >= cus && (int64_t)len * 4 * D <= 2 * kOneSplitBytes) return 1;
   const int most = most_splits_for(units, D, len, cus), by_len = (len + kMaxChunk - 1) / kMaxChunk;
   int s = (int)(cus / units);
@@ -146,9 +152,8 @@ int default_splits_for(int rows, int NKV, int D, int len, int cus) {
     const int longest = s > by_len ? s : by_len;
     s = two < longest ? two : longest;
   }
-  int merged = kb / 32 < 2 * kMergeBatch ? (int)(kb / 32) : 2 * kMergeBatch;
-  if (merged < kMergeBatch) merged = kMergeBatch;
-  if (merged < (kb + 127) / 128) merged = (int)((kb + 127) / 128);
+  const int second = raised(kMergeBatch, 32);
+  const int merged = raised(second < 2 * kMergeBatch ? second : 2 * kMergeBatch, 128);
   if (s > merged) s = merged;
   if (s > most) s = most;
   return s < 1 ? 1 : s;

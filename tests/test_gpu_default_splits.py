@@ -15,7 +15,10 @@ CASES = [
     (2, 16, 8, 128, 2048, 16),    # one round: 256 workgroups
     (3, 16, 8, 128, 2000, 10),    # one round, rounded down: 240
     (1, 8, 1, 128, 1000, 16),     # the merge batch bounds a single unit
-    (1, 8, 1, 128, 1300, 20),     # ... a second batch for chunks of 64 positions
+    (1, 8, 1, 128, 1300, 21),     # ... a second batch for chunks of 64 positions, none of 65
+    (1, 16, 8, 128, 1500, 24),
+    (1, 8, 1, 128, 1087, 16),     # ... but no second batch for less than 17 whole chunks
+    (1, 8, 1, 128, 8450, 34),     # ... chunks of 256 positions, none of 257
     (1, 8, 1, 128, 4000, 32),     # ... two batches
     (1, 8, 1, 128, 9000, 36),     # ... more for chunks of 256 positions
     (1, 8, 1, 64, 9000, 32),      # (512 at head_dim 64)
