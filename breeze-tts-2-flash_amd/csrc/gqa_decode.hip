@@ -103,7 +103,7 @@ int effective_len(int capacity, int max_seq_len) {
 // (the kernels apply the same bound to each row's actual length): the cross-workgroup merge of two or more splits costs
 // about 2 us, more than one workgroup takes to stream 64 KB (cold, B2 16/8: head_dim 128, 128 positions 4.45 against
 // 5.42 us; head_dim 64, 256 positions 4.47 against 5.17; at 128 KB one split is slower: 6.23 against 5.47). The static
-// scratch refuses by this bound and a workspace is sized for it, so neither follows the tuning below.
+// scratch refuses by this bound and a workspace is sized for it, so what they take does not follow the tuning below.
 constexpr int kMaxChunk = 256;
 
 int most_splits_for(int64_t units, int D, int len, int cus) {
@@ -191,12 +191,7 @@ int check_sizes(int B, int NH, int NKV, int D, int cap) {
 int tokens_of(const bz_gqa_decode_args* a) { return a->tokens_per_row > 1 ? a->tokens_per_row : 1; }
 int rows_of(const bz_gqa_decode_args* a) { return a->batch * tokens_of(a); }
 
-// step: a fused call with lengths. Up to kStepRows rows over up to kStepLen positions (a backbone decode step) it keeps
-// most_splits_for, the count it always had: another count changes the order of the sums, which travels through the
-// step's later layers (see use_mfma).
-constexpr int kStepRows = 4, kStepLen = 4096;
-
-int resolve_splits(const bz_gqa_decode_args* a, bool step, int* splits) {
+int resolve_splits(const bz_gqa_decode_args* a, int* splits) {
   if (a->num_splits < 0 || a->num_splits > kMaxSplits) return BZ_ERR_SHAPE;
   if (a->num_splits > 0) {
     *splits = a->num_splits;
@@ -205,11 +200,8 @@ int resolve_splits(const bz_gqa_decode_args* a, bool step, int* splits) {
   int cus = 0;
   const int rc = device_cus(&cus);
   if (rc != BZ_OK) return rc;
-  const int rows = rows_of(a), len = effective_len(a->capacity, a->max_seq_len);
-  if (step && rows <= kStepRows && len <= kStepLen)
-    *splits = most_splits_for((int64_t)rows * a->num_kv_heads, a->head_dim, len, cus);
-  else
-    *splits = default_splits_for(rows, a->num_kv_heads, a->head_dim, len, cus);
+  *splits = default_splits_for(rows_of(a), a->num_kv_heads, a->head_dim, effective_len(a->capacity, a->max_seq_len),
+                               cus);
   return BZ_OK;
 }
 
@@ -329,7 +321,7 @@ int launch(const bz_gqa_decode_args* a, hipStream_t stream, const int32_t* seq_l
   if (mask_kind == BZ_MASK_NONE && seq_lens == nullptr) return BZ_ERR_NULL;
   if (seq_lens != nullptr && wave_route(a, mask_kind, f)) return launch_wave(a, stream, seq_lens, kv_start);
   int splits = 0;
-  int rc = resolve_splits(a, f != nullptr && mask_kind == BZ_MASK_NONE, &splits);
+  int rc = resolve_splits(a, &splits);
   if (rc != BZ_OK) return rc;
   WsLayout ws;
   char* wsb = nullptr;
@@ -584,7 +576,7 @@ __attribute__((visibility("default"))) int bz_gqa_decode_workspace_size(int32_t 
     int cus = 0;
     rc = device_cus(&cus);
     if (rc != BZ_OK) return rc;
-    // of every default count (a fused step's can be higher than bz_gqa_decode's)
+    // the bound of every default count: a size that does not follow their tuning
     splits = most_splits_for((int64_t)batch * num_kv_heads, head_dim, effective_len(capacity, max_seq_len), cus);
   }
   *bytes = ws_layout(batch, num_q_heads, num_kv_heads, head_dim, splits).total;

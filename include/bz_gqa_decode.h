@@ -125,12 +125,13 @@ int bz_gqa_decode(const bz_gqa_decode_args* args, hipStream_t stream);
    forbid allocation. With args->seq_lens NULL the range of each row comes from args->mask, as in
    bz_gqa_decode_masked. Limits: at most 1024 (row, kv head) groups (batch * tokens_per_row * num_kv_heads) and
    8 MiB of split partials (batch * tokens_per_row * num_q_heads * splits * (head_dim + 2) * 4 bytes), else
-   BZ_ERR_SCRATCH. Every call on a device shares that device's scratch: calls that overlap in time on one device
+   BZ_ERR_SCRATCH. With num_splits 0 the limit counts the splits that bz_gqa_decode_workspace_size sizes for: one
+   workgroup per CU or one split per 256 positions, whichever is more, whatever default is taken. Every call on a device shares that device's scratch: calls that overlap in time on one device
    (several streams, several host threads) race and must be ordered by the caller. */
 int bz_gqa_decode_noalloc(const bz_gqa_decode_args* args, hipStream_t stream);
 
-/* Bytes of workspace bz_gqa_decode needs for these sizes (num_splits as passed, 0 = default; with tokens_per_row
-   T > 1 pass batch * T). Replaces the caller-side sizing of the reference's scores/cmax/part/counters buffers
+/* Bytes of workspace bz_gqa_decode needs for these sizes (num_splits as passed, 0 = default: at least as many as
+   bz_gqa_decode_default_splits; with tokens_per_row T > 1 pass batch * T). Replaces the caller-side sizing of the reference's scores/cmax/part/counters buffers
    (flash/backbone.py:27-37). */
 int bz_gqa_decode_workspace_size(int32_t batch, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
                                  int32_t capacity, int32_t num_splits, int32_t max_seq_len, size_t* bytes);

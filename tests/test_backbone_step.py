@@ -146,3 +146,11 @@ def test_install_declines_other_gpus(monkeypatch, capsys):
     assert backbone.install(_Declined) is False
     assert _Declined._decode_step is before
     assert "not installed: Fake GPU" in capsys.readouterr().out
+
+
+# rows, kv heads, cache slots, splits on 256 CUs: each bound of the count, and the library's default past 4096 slots
+@pytest.mark.parametrize("rows,kv_heads,length,splits", [(2, 8, 2048, 16), (1, 8, 2048, 32), (3, 8, 2000, 11), (4, 8, 4096, 16),
+                                                         (1, 1, 4000, 125), (1, 1, 4096, 128), (2, 8, 128, 1), (2, 8, 129, 5),
+                                                         (2, 8, 4097, 0)])
+def test_step_split_count(rows, kv_heads, length, splits):
+    assert backbone.step_splits(rows, kv_heads, length, 256) == splits

@@ -59,24 +59,22 @@ def test_static_scratch_refuses_by_the_largest_default(device):
     assert rc == 0
 
 
-@pytest.mark.parametrize("B,NKV,G,cap", [(1, 4, 4, 4096), (2, 8, 4, 2048), (4, 8, 2, 3000), (5, 2, 4, 1024), (1, 4, 1, 5000)])
-def test_a_step_keeps_its_bits(device, B, NKV, G, cap):
-    """A fused call with lengths of up to four rows and 4096 positions runs one split per 256 positions or one workgroup
-    per CU, whichever is more (at least 32 positions each); any other takes the tuned count. One workspace of the
-    default size serves both."""
+@pytest.mark.parametrize("B,NKV,G,cap", [(1, 1, 2, 4000), (1, 4, 4, 4096), (2, 8, 4, 2048), (4, 8, 2, 3000), (5, 2, 4, 1024),
+                                         (1, 4, 1, 5000)])
+def test_fused_default_is_the_queried_count(device, B, NKV, G, cap):
+    """bz_gqa_decode_default_splits is what num_splits = 0 takes in the fused call as well: a workspace sized for that count
+    serves it, and its outputs equal the explicit count's bit for bit."""
     from tests.test_gpu_fused import make_step, tens
 
-    cus = torch.cuda.get_device_properties(device).multi_processor_count
-    step = B <= 4 and cap <= 4096
-    old = min(max(-(-cus // (B * NKV)), -(-cap // 256)), -(-cap // 32), 256)
-    splits = old if step else default_splits(B, NKV, 128, cap)
-    assert workspace_bytes(B, NKV * G, NKV, 128, cap) == workspace_bytes(B, NKV * G, NKV, 128, cap, old)
+    splits = default_splits(B, NKV, 128, cap)
+    ws = torch.zeros(workspace_bytes(B, NKV * G, NKV, 128, cap, splits), dtype=torch.uint8, device=device)
     s = make_step(cap, B=B, NH=NKV * G, NKV=NKV, cap=cap, pos=cap - 5)
     lens = torch.full((B,), cap - 4, dtype=torch.int32, device=device)
     outs = []
     for n in (0, splits):
         outs.append(gqa_decode_fused(*(tens(s[k], device) for k in ("qkv", "qn", "kn")), 1e-6, tens(s["cos"], device),
                                      tens(s["sin"], device), tens(s["kc"], device), tens(s["vc"], device),
-                                     torch.tensor([cap - 5], device=device), 128 ** -0.5, seq_lens=lens, num_splits=n))
+                                     torch.tensor([cap - 5], device=device), 128 ** -0.5, seq_lens=lens, num_splits=n,
+                                     workspace=ws))
     torch.cuda.synchronize()
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
