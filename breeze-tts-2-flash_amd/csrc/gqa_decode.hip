@@ -67,8 +67,7 @@ int min_chunk_for(int D) { return (16 * 1024) / (4 * D); }
 // Positions per thread per tile: 1 when two one-position tiles cover the expected chunk, else 2. Two tiles (A, B) are
 // in flight from the start, so the first tile's arithmetic overlaps the second tile's arrival. Tiles of more
 // positions (4 was measured) leave more arithmetic exposed after the last tile arrives: config 3 +2%, config 4 +6%.
-int ppt_for(int D, int G, int chunk, int nt) {
-  (void)G;
+int ppt_for(int D, int chunk, int nt) {
   const int rows = nt / (D / 8);
   return 2 * rows >= chunk ? 1 : 2;
 }
@@ -359,7 +358,7 @@ int launch(const bz_gqa_decode_args* a, hipStream_t stream, const int32_t* seq_l
   int chunk = (len + splits - 1) / splits;
   if (chunk < min_chunk) chunk = min_chunk;
   const int nt = kSplitThreads;
-  const int ppt = ppt_for(D, G, chunk, nt);
+  const int ppt = matrix && !vector_short(G, mask_kind, f != nullptr, splits, len) ? kMatrix : ppt_for(D, chunk, nt);
   SplitFn split_fn = pick_split(D, G, mask_kind, ppt, nt, f != nullptr);
   CombineFn comb_fn = pick_combine(D, G, matrix);
   if (split_fn == nullptr || comb_fn == nullptr) return BZ_ERR_UNSUPPORTED;

@@ -673,6 +673,15 @@ __device__ __forceinline__ void consume_tile(Tile<PPT>& t, const uint4 (&qp)[G],
 // rounding in one layer's attention travels through every later layer of a step (28 layers: 1.7% in the logits from 1e-5 in
 // each call), and a step's results stay what they were, bit for bit.
 constexpr bool use_mfma(int G, int MK, bool FUSED) { return G == 8 || (G == 4 && !(FUSED && MK == BZ_MASK_NONE)); }
+// A chunk of one or two of the vector path's one-position tiles ends before the matrix tiles' LDS hand-over of 3 G columns
+// pays (G 4, no mask, one split, us per call over 9 / 17 / 32 / 64 positions, vector / matrix: D 128 3.10 / 3.40, 3.42 /
+// 3.40, 3.44 / 3.43, 3.81 / 3.57; D 64 2.85 / 3.02, 2.85 / 3.01, 2.85 / 3.01, 3.18 / 3.04). With a mask the scan hides most of
+// it (D 128 4.43 / 4.56 over 9 positions, 4.78 / 4.62 over 17; D 64 4.13 / 3.93), and with more splits the matrix tiles'
+// merge wins (16 chunks of 32 positions 5.92 / 5.34); G 8 with a mask: 6.41 / 4.73 over 17 positions.
+constexpr bool vector_short(int G, int mk, bool fused, int splits, int len) {
+  return G == 4 && mk == BZ_MASK_NONE && !fused && splits == 1 && len <= 32;
+}
+constexpr int kMatrix = 0;  // in the place of PPT
 
 // With four or more q heads per kv head the dot products are a contraction for the matrix cores: the vector path above
 // spends about 70 G VALU instructions per 16 positions and wave (dot2, DPP row sums, an fma per head and dim; at G = 8
@@ -851,12 +860,12 @@ __device__ __forceinline__ void consume_wave_tile(WaveTile<D>& t, const bf16x8_t
 // ---------------------------------------------------------------------------------------------- kernels
 
 // lens, starts: p.seq_lens and p.kv_start again, as leading (preloaded) arguments.
-// MX: the tiles go through the matrix cores (use_mfma). The bound on registers there keeps the accumulators out
-// of AGPRs, which the rescaling would have to move to and fro.
+// PPT: positions per thread and tile of the vector path; kMatrix (0, MX below): the tiles go through the matrix cores.
+// The bound on registers there keeps the accumulators out of AGPRs, which the rescaling would have to move to and fro.
 template <int D, int G, int PPT, int MK, int NT, bool FUSED>
-__global__ void __launch_bounds__(NT, use_mfma(G, MK, FUSED) ? (D == 128 ? 2 : 3) : 1)
+__global__ void __launch_bounds__(NT, PPT == kMatrix ? (D == 128 ? 2 : 3) : 1)
     gqa_split_kernel(const int32_t* lens, const int32_t* starts, const int tpr, const Params p) {
-  constexpr bool MX = use_mfma(G, MK, FUSED);
+  constexpr bool MX = PPT == kMatrix;
   constexpr int NW = NT / kWave;               // waves per workgroup
   constexpr int LPR = D / 8;                   // lanes per KV row, 16 B (8 bf16) each
   constexpr int ROWS = NT / LPR;               // KV rows per load instruction across the workgroup
@@ -1324,9 +1333,15 @@ __global__ void __launch_bounds__(kThreads) gqa_probs_kernel(const Params p, flo
 
 template <int D, int G, int MK, int NT, bool FUSED>
 SplitFn pick_ppt(int ppt) {
-  if constexpr (!use_mfma(G, MK, FUSED))
+  if constexpr (use_mfma(G, MK, FUSED)) {
+    if (ppt == kMatrix) return gqa_split_kernel<D, G, kMatrix, MK, NT, FUSED>;
+    if constexpr (G == 4 && MK == BZ_MASK_NONE)  // vector_short
+      if (ppt == 1) return gqa_split_kernel<D, G, 1, MK, NT, FUSED>;
+  } else {
+    if (ppt == 1) return gqa_split_kernel<D, G, 1, MK, NT, FUSED>;
     if (ppt == 2) return gqa_split_kernel<D, G, 2, MK, NT, FUSED>;
-  return gqa_split_kernel<D, G, 1, MK, NT, FUSED>;  // the matrix tiles have one form
+  }
+  return nullptr;
 }
 
 template <int D, int G, int NT, bool FUSED>

@@ -30,6 +30,24 @@ def test_lengths_around_the_tiles(device, D, NH, NKV, splits):
     assert_close(out.float().cpu().numpy(), oracle(w, kv_start=starts), f"D={D} G={NH // NKV} splits={splits}")
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("cap", [1, 17, 32, 33])
+def test_one_short_split_of_a_group_of_four(device, D, cap):
+    """One split of at most 32 positions takes the vector path, 33 the matrix tiles; a max_seq_len below the capacity
+    counts, and lengths beyond it stay right."""
+    lens = list(range(1, cap + 1))
+    w, _ = rand_case(cap + D, cap, 8, 2, D, cap, lens)
+    ref = oracle(w)
+    for b, n in enumerate(lens):
+        w.k[b, :, n:] = w.v[b, :, n:] = float("nan")
+    g = w.to(device)
+    for msl in (0, 7):
+        for combine in ("auto", "kernel"):
+            out = gqa_decode(g.q, g.k, g.v, g.seq_lens, g.scale, num_splits=1, max_seq_len=msl, combine=combine)
+            torch.cuda.synchronize()
+            assert_close(out.float().cpu().numpy(), ref, f"D={D} cap={cap} max_seq_len={msl} {combine}")
+
+
 @pytest.mark.parametrize("NH,NKV", GROUPS)
 def test_probabilities_keep_their_low_bits(device, NH, NKV):
     """V is +1 at one position and -1 at another whose score differs by d: the result tanh(d / 2) is the difference of
