@@ -856,10 +856,31 @@ GemvFn pick_block(int m, int k, int ntot, int epi, bool norm, int cus, int* thre
   return m == 3 ? pick_block_m<3, 256>(eight, epi, norm) : pick_block_m<4, 256>(eight, epi, norm);
 }
 
+// Workgroups of q quads (outputs of SiLU * up: q / 2) over the CUs. g is even where its last round is 90% full; where it is
+// one round that twice as many, smaller workgroups would exceed; or from four rounds on, past k = 3072 (four chunks a wave,
+// where two quads cost more) one and a half with the last 75% full.
+struct Quads {
+  int quads, cus, k;
+  bool silu;
+  int groups(int q) const { return (quads + (silu ? q / 2 : q) - 1) / (silu ? q / 2 : q); }
+  int rounds(int g) const { return (g + cus - 1) / cus; }
+  bool full(int g, int tenths) const { return 10 * (int64_t)g >= (int64_t)tenths * cus * rounds(g); }
+  bool even(int g) const {
+    if (full(g, 9) || (g <= cus && 2 * g > cus)) return true;
+    return k > 3072 ? 2 * (int64_t)g > 3 * (int64_t)cus && 4 * (int64_t)g >= 3 * (int64_t)cus * rounds(g) : g >= 4 * cus;
+  }
+};
+Quads quads_of(int k, int n0, int n1, int n2, bool silu, int cus) {
+  return {(n0 + 3) / 4 + (silu ? 0 : (n1 + 3) / 4 + (n2 + 3) / 4), cus, k, silu};
+}
+
 // Where the 4x4x4 MFMA kernel is taken (graph of calls on their own weights, us per call, the other kernels -> this one):
 //   SiLU * up for 2048 < k <= 4096 (x in LDS before), M = 1 / 2 / 4: k 4096, 12288 outputs 41.1 / 42.2 / 47.1 -> 31.8 / 30.8 /
 //     32.9 (6.5 TB/s); 3072, 8192: 19.6 / 20.6 / 23.1 -> 17.8 / 17.7 / 18.2; 2976, 4960: 16.8 / 16.8 / 19.2 -> 12.7 / 12.5 /
-//     13.7; 2560, 6912: 16.1 / 16.2 / 19.0 -> 14.6 / 15.1 / 16.8;
+//     13.7; 2560, 6912: 16.1 / 16.2 / 19.0 -> 14.6 / 15.1 / 16.8. Past k = 3072 not at M <= 2 where this kernel's second or
+//     fourth round is 75 to 90% full, as the LDS kernel's last round is too (its workgroup has as many outputs or twice as
+//     many): k 3840, 6912 outputs, M = 1 / 2: 19.6 / 20.1, here 20.9 / 21.5; and at M = 1 not where a single round is between
+//     half and three quarters full: k 3840, 1152 outputs 6.1, here 6.8;
 //   plain there at M >= 3: k 4096, 6144 rows 11.8 / 13.0 -> 11.5 / 12.0 at M = 3 / 4 (M = 1 / 2: 10.7 / 11.1 against 12.4 /
 //     12.6);
 //   at M = 3 also SiLU * up up to k = 1024 (1024, 3072 outputs 5.3 -> 4.5; 512, 1536 3.3 -> 3.2), plain there past 2048
@@ -868,10 +889,15 @@ GemvFn pick_block(int m, int k, int ntot, int epi, bool norm, int cus, int* thre
 //     layer travels through the later ones, and the sizes a step has (hidden sizes up to 2048) keep their bits: at M = 4 the
 //     block kernel is level there (k 2048, 6144 outputs 10.3 either way).
 // Up to k = 256 half of its waves would idle.
-bool mfma_route(int m, int k, int rows, int epi) {
+bool mfma_route(int m, int k, int rows, int epi, const Quads& t) {
   if (k <= 256 || k > 4096) return false;
   const bool three = m == 3 && k <= 1024;
-  if (epi == BZ_GEMV_SILU_MUL) return k > 2048 || three;
+  if (epi == BZ_GEMV_SILU_MUL) {
+    const int g = t.groups(4), rounds = t.rounds(g);
+    if (m <= 2 && k > 3072 && (rounds == 2 || rounds == 4) && !t.full(g, 9) && 4 * g >= 3 * t.cus * rounds) return false;
+    if (m == 1 && k > 3072 && 2 * g > t.cus && 4 * g < 3 * t.cus) return false;
+    return k > 2048 || three;
+  }
   if (epi == BZ_GEMV_PLAIN) return k > 2048 ? m >= 3 : three && rows > 2048;
   return k > 2048 && m == 3;
 }
@@ -893,21 +919,16 @@ GemvFn pick_mfma_q(int q, int epi, bool norm) {
   return pick_mfma_epi<NW, TR, 1>(epi, norm);
 }
 
-// Four waves up to k = 1024 (one or two chunks each), eight above. Quads per workgroup: the most whose grid fills its
-// last round of CUs to 90% or is long enough (four rounds) for that not to matter; else two, or one where two leave CUs
-// without a workgroup (us per call, 4 / 2 quads: plain at k 4096, 384 / 768 workgroups 12.9 / 12.0; k 2048, 256 / 512: 5.1
-// / 5.7; gate / up at k 2976, 620 / 1240: 13.5 / 12.6; k 2048, 768 / 1536: 10.3 / 11.6; residual at k 3072, 1024 rows: 2
-// quads 3.8, 1 3.3).
-GemvFn pick_mfma(int k, int n0, int n1, int n2, int epi, bool norm, int cus, int* threads, int* grid) {
-  const bool silu = epi == BZ_GEMV_SILU_MUL;
-  const int quads = (n0 + 3) / 4 + (silu ? 0 : (n1 + 3) / 4 + (n2 + 3) / 4);
+// Four waves up to k = 1024 (one or two chunks each), eight above. Quads per workgroup: four where their grid is even, else
+// two, or one where two leave CUs without a workgroup (us per call, 4 / 2 quads: plain at k 4096, 384 / 768 workgroups 12.9 /
+// 12.0, k 3584, 640 / 1280 16.0 / 17.6; gate / up at k 2976, 620 / 1240 13.5 / 12.6, k 3328, 864 / 1728 19.7 / 22.8, 608 / 1216
+// 14.7 / 16.6, k 2560, 144 / 288 5.8 / 6.3; residual at k 3072, 1024 rows: 2 quads 3.8, 1 3.3).
+GemvFn pick_mfma(int k, const Quads& t, int epi, bool norm, int* threads, int* grid) {
   const int nw = k <= 1024 ? 4 : 8;
-  auto groups = [&](int q) { return (quads + (silu ? q / 2 : q) - 1) / (silu ? q / 2 : q); };
-  auto even = [&](int g) { return g >= 4 * cus || 10 * (int64_t)g >= 9 * (int64_t)cus * ((g + cus - 1) / cus); };
   int q = 4;
-  if (!even(groups(4))) q = silu || groups(2) >= cus ? 2 : 1;
+  if (!t.even(t.groups(4))) q = t.silu || t.groups(2) >= t.cus ? 2 : 1;
   *threads = nw * kWave;
-  *grid = groups(q);
+  *grid = t.groups(q);
   switch (nw == 4 ? (k <= 512 ? 1 : 2) : 10 * ((k + 1023) / 1024)) {  // chunks per wave (mfma_route: no k in 1025..2048)
     case 1: return pick_mfma_q<4, 1>(q, epi, norm);
     case 2: return pick_mfma_q<4, 2>(q, epi, norm);
@@ -988,9 +1009,9 @@ __attribute__((visibility("default"))) int bz_gemv(const bz_gemv_args* a, hipStr
   int cus = 0;
   const int rc = bz::device_cu_count(&cus);
   if (rc != BZ_OK) return rc;
-  if (mfma_route(a->m, a->k, ntot, a->epilogue)) {
-    GemvFn mf = pick_mfma(a->k, p.n0, p.n1, ntot - p.n0 - p.n1, a->epilogue, a->norm_weight != nullptr, cus, &bthreads,
-                          &bgrid);
+  const Quads quads = quads_of(a->k, p.n0, p.n1, ntot - p.n0 - p.n1, a->epilogue == BZ_GEMV_SILU_MUL, cus);
+  if (mfma_route(a->m, a->k, ntot, a->epilogue, quads)) {
+    GemvFn mf = pick_mfma(a->k, quads, a->epilogue, a->norm_weight != nullptr, &bthreads, &bgrid);
     if (mf == nullptr) return BZ_ERR_UNSUPPORTED;
     hipLaunchKernelGGL(mf, dim3(bgrid), dim3(bthreads), 0, stream, p.w0, p.w1, p.w2, p.n0, p.n1, p.ntot,
                        p.k | a->m << 24, p.x, p.ldx, p);

@@ -15,7 +15,12 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("M,K,N", [(3, 264, 9), (3, 512, 70), (3, 520, 1030), (3, 1024, 64), (3, 1032, 515), (3, 2048, 2050),
                                    (1, 2056, 33), (2, 2176, 1100), (4, 3072, 514), (2, 3080, 130), (1, 4096, 2052),
-                                   (4, 4088, 1026)])
+                                   (4, 4088, 1026),
+                                   # four quads a workgroup (256 CUs): one round, its edge, many rounds, the last ragged
+                                   (2, 2056, 2046), (4, 2304, 1031), (1, 2816, 2043), (3, 3584, 6913), (2, 4096, 8199),
+                                   (4, 3080, 5001),
+                                   # two quads: a grid just past a round of four; the LDS kernel's sizes between
+                                   (2, 2304, 3001), (4, 3328, 2307), (1, 3328, 3331), (2, 3840, 6917), (1, 4096, 1283)])
 def test_gateup(device, M, K, N):
     rng = np.random.default_rng(M * K + N)
     x, nw = rand_bits(rng, M, K), f32_to_bf16((1 + 0.2 * rng.standard_normal(K)).astype(np.float32))
@@ -28,7 +33,10 @@ def test_gateup(device, M, K, N):
 
 @pytest.mark.parametrize("norm", [True, False])
 @pytest.mark.parametrize("M,K,ns", [(3, 568, (2049, 6, 3)), (3, 2048, (1030, 513, 517)), (4, 2056, (13, 7, 30)),
-                                    (3, 3000, (5, 1, 2)), (4, 4096, (1024, 512, 512)), (3, 4096, (1, 0, 0))])
+                                    (3, 3000, (5, 1, 2)), (4, 4096, (1024, 512, 512)), (3, 4096, (1, 0, 0)),
+                                    # four quads a workgroup, ragged segments: one round, two and a half past k = 3072
+                                    (4, 2056, (1030, 513, 517)), (3, 3072, (2049, 1022, 1001)), (3, 3584, (5121, 2563, 2553)),
+                                    (4, 2560, (2001, 1603, 1602))])  # two quads
 def test_segments(device, M, K, ns, norm):
     rng = np.random.default_rng(M * K + sum(ns))
     x = rand_bits(rng, M, K)
