@@ -20,7 +20,7 @@
 // a block-ordered kernel runs instead: a workgroup streams its rows as one contiguous block, every thread holding one
 // x vector for all of its rows, and the sums are reduced over the workgroup once, at the end (gemv_block_kernel).
 // A third kernel works the products out on the 4x4x4 MFMA, four weight rows per load (gemv_mfma_kernel): for
-// 2048 < k <= 4096 and for M = 3 (mfma_route).
+// 2048 < k <= 4096, most of SiLU * up and plain at M >= 3 (mfma_route).
 #include <hip/hip_runtime.h>
 
 #include <math.h>
@@ -537,18 +537,22 @@ __global__ void __launch_bounds__(NT)
 // Against four dot2 per vector and row of x on the vector unit (the kernels above) that is an eighth of the instructions
 // at four rows of x, where they bound the tail of every workgroup.
 //
-// A workgroup of NW waves owns Q such groups of four rows ("quads"; with the SiLU * up epilogue the first half are gate
-// quads, the second the up quads of the same outputs) and splits k over its waves: wave w takes the TR chunks w, w + NW,
-// ..., so that the workgroup reads NW * 256 consecutive bytes of every row at a time, x once, and every load goes out at
+// A workgroup of eight waves owns Q such groups of four rows ("quads"; with the SiLU * up epilogue the first half are gate
+// quads, the second the up quads of the same outputs) and splits k over its waves: wave w takes the TR chunks w, w + 8,
+// ..., so that the workgroup reads 2048 consecutive bytes of every row at a time, x once, and every load goes out at
 // once. Each weight segment starts a quad of its own, so a quad has one resource, cut at its last row; lanes past k take
 // an offset outside of it (their loads read 0: a neighbouring row's Inf or NaN must not meet x's padding). The sums meet
 // in LDS.
-template <int Q, int NW, int TR, bool NORM, int EPI>
-__global__ void __launch_bounds__(NW* kWave)
+constexpr int kMfmaWaves = 8;
+
+template <int Q, int TR, bool NORM, int EPI>
+__global__ void __launch_bounds__(kMfmaWaves* kWave)
     gemv_mfma_kernel(const uint16_t* w0, const uint16_t* w1, const uint16_t* w2, int n0, int n1, int ntot, int km,
                      const uint16_t* x, int64_t ldx, const GemvParams p) {
   constexpr bool SILU = EPI == BZ_GEMV_SILU_MUL;
   constexpr int QO = SILU ? Q / 2 : Q;  // quads of outputs
+  constexpr int NW = kMfmaWaves;
+  static_assert(EPI != BZ_GEMV_RESIDUAL, "the residual epilogue stays on the other kernels");
   constexpr uint32_t kOut = 0x40000000u;  // past every quad (4 k * 2 bytes)
   const int k = km & 0xffffff, M = km >> 24;  // one preloaded argument
   const int tid = threadIdx.x, lane = tid % kWave, wave = wave_uniform(tid / kWave);
@@ -604,12 +608,6 @@ __global__ void __launch_bounds__(NW* kWave)
   const bool writes = tid < kWave && (Q == 4 || (tid & (Q == 2 ? 4 : 12)) == 0) && vq < QO && j < M;
   int row = 0, rows = 0;
   if (tid < kWave) (void)quad(vq, false, row, rows);
-  float resv = 0.f;
-  if (EPI == BZ_GEMV_RESIDUAL) {
-    const Rsrc rr = span_rsrc(p.res, (int)(((int64_t)(M - 1) * p.ldr + ntot) * 2));
-    const uint32_t off = writes && vr < rows ? (uint32_t)((j * p.ldr + row + vr) * 2) : 0xfffffff0u;
-    resv = bf16_to_f32(__builtin_amdgcn_raw_buffer_load_b16(rr, off, 0, 0));
-  }
   __builtin_amdgcn_sched_barrier(0);
 
   if (NORM) {
@@ -699,8 +697,6 @@ __global__ void __launch_bounds__(NW* kWave)
   float out;
   if (EPI == BZ_GEMV_PLAIN) {
     out = red;
-  } else if (EPI == BZ_GEMV_RESIDUAL) {
-    out = resv + bf16_to_f32(f32_to_bf16(red));
   } else {
     const float gt = bf16_to_f32(f32_to_bf16(red));
     const float u = bf16_to_f32(f32_to_bf16(upv));
@@ -883,59 +879,43 @@ Quads quads_of(int k, int n0, int n1, int n2, bool silu, int cus) {
 //     half and three quarters full: k 3840, 1152 outputs 6.1, here 6.8;
 //   plain there at M >= 3: k 4096, 6144 rows 11.8 / 13.0 -> 11.5 / 12.0 at M = 3 / 4 (M = 1 / 2: 10.7 / 11.1 against 12.4 /
 //     12.6);
-//   at M = 3 also SiLU * up up to k = 1024 (1024, 3072 outputs 5.3 -> 4.5; 512, 1536 3.3 -> 3.2), plain there past 2048
-//     rows (568, 2560 rows 3.9 -> 3.1) and the residual for 2048 < k <= 4096 (3072, 1024 rows 4.0 -> 3.5). M = 1, 2 and 4
-//     are the rows of a backbone decode step: one stream, a CFG pair, two pairs. There another order of the sums in one
-//     layer travels through the later ones, and the sizes a step has (hidden sizes up to 2048) keep their bits: at M = 4 the
-//     block kernel is level there (k 2048, 6144 outputs 10.3 either way).
-// Up to k = 256 half of its waves would idle.
-bool mfma_route(int m, int k, int rows, int epi, const Quads& t) {
-  if (k <= 256 || k > 4096) return false;
-  const bool three = m == 3 && k <= 1024;
-  if (epi == BZ_GEMV_SILU_MUL) {
-    const int g = t.groups(4), rounds = t.rounds(g);
-    if (m <= 2 && k > 3072 && (rounds == 2 || rounds == 4) && !t.full(g, 9) && 4 * g >= 3 * t.cus * rounds) return false;
-    if (m == 1 && k > 3072 && 2 * g > t.cus && 4 * g < 3 * t.cus) return false;
-    return k > 2048 || three;
-  }
-  if (epi == BZ_GEMV_PLAIN) return k > 2048 ? m >= 3 : three && rows > 2048;
-  return k > 2048 && m == 3;
+// Up to k = 2048 it measured faster at four rows too (SiLU * up at k 1024, 3072 outputs 6.0 -> 4.6; 568, 2272 5.9 -> 3.8; level
+// with the block kernel at 2048, 6144). Every M keeps the other kernels there: a backbone step of such a hidden size is held
+// to 1% of its earlier outputs, and another order of the sums in one layer, no less exact, moves them by up to 1.5% after 12
+// layers (use_mfma in gqa_kernels.cuh has the figures). A step of a hidden size above 2048 does change: its MLP gains a
+// quarter. The residual epilogue gains 12% at k 4096, 1024 rows and loses 7% at k 3072, 1536: it stays on the other kernels.
+bool mfma_route(int m, int k, int epi, const Quads& t) {
+  if (k <= 2048 || k > 4096) return false;
+  if (epi == BZ_GEMV_PLAIN) return m >= 3;
+  if (epi != BZ_GEMV_SILU_MUL) return false;
+  const int g = t.groups(4), rounds = t.rounds(g);
+  if (m <= 2 && k > 3072 && (rounds == 2 || rounds == 4) && !t.full(g, 9) && 4 * g >= 3 * t.cus * rounds) return false;
+  return !(m == 1 && k > 3072 && 2 * g > t.cus && 4 * g < 3 * t.cus);
 }
 
-template <int NW, int TR, int Q>
-GemvFn pick_mfma_epi(int epi, bool norm) {
-  if (epi == BZ_GEMV_PLAIN)
-    return norm ? gemv_mfma_kernel<Q, NW, TR, true, BZ_GEMV_PLAIN> : gemv_mfma_kernel<Q, NW, TR, false, BZ_GEMV_PLAIN>;
-  if (epi == BZ_GEMV_RESIDUAL) return norm ? nullptr : gemv_mfma_kernel<Q, NW, TR, false, BZ_GEMV_RESIDUAL>;
+template <int TR, int Q>
+GemvFn pick_mfma_epi(bool silu, bool norm) {
+  if (!silu) return norm ? gemv_mfma_kernel<Q, TR, true, BZ_GEMV_PLAIN> : gemv_mfma_kernel<Q, TR, false, BZ_GEMV_PLAIN>;
   if constexpr (Q > 1)
-    return norm ? gemv_mfma_kernel<Q, NW, TR, true, BZ_GEMV_SILU_MUL>
-                : gemv_mfma_kernel<Q, NW, TR, false, BZ_GEMV_SILU_MUL>;
+    return norm ? gemv_mfma_kernel<Q, TR, true, BZ_GEMV_SILU_MUL> : gemv_mfma_kernel<Q, TR, false, BZ_GEMV_SILU_MUL>;
   return nullptr;
 }
-template <int NW, int TR>
-GemvFn pick_mfma_q(int q, int epi, bool norm) {
-  if (q == 4) return pick_mfma_epi<NW, TR, 4>(epi, norm);
-  if (q == 2) return pick_mfma_epi<NW, TR, 2>(epi, norm);
-  return pick_mfma_epi<NW, TR, 1>(epi, norm);
+template <int TR>
+GemvFn pick_mfma_q(int q, bool silu, bool norm) {
+  if (q == 4) return pick_mfma_epi<TR, 4>(silu, norm);
+  if (q == 2) return pick_mfma_epi<TR, 2>(silu, norm);
+  return pick_mfma_epi<TR, 1>(silu, norm);
 }
 
-// Four waves up to k = 1024 (one or two chunks each), eight above. Quads per workgroup: four where their grid is even, else
-// two, or one where two leave CUs without a workgroup (us per call, 4 / 2 quads: plain at k 4096, 384 / 768 workgroups 12.9 /
-// 12.0, k 3584, 640 / 1280 16.0 / 17.6; gate / up at k 2976, 620 / 1240 13.5 / 12.6, k 3328, 864 / 1728 19.7 / 22.8, 608 / 1216
-// 14.7 / 16.6, k 2560, 144 / 288 5.8 / 6.3; residual at k 3072, 1024 rows: 2 quads 3.8, 1 3.3).
-GemvFn pick_mfma(int k, const Quads& t, int epi, bool norm, int* threads, int* grid) {
-  const int nw = k <= 1024 ? 4 : 8;
+// Quads per workgroup: four where their grid is even, else two, or one where two leave CUs without a workgroup (us per call,
+// 4 / 2 quads: plain at k 4096, 384 / 768 workgroups 12.9 / 12.0, k 3584, 640 / 1280 16.0 / 17.6; gate / up at k 2976, 620 /
+// 1240 13.5 / 12.6, k 3328, 864 / 1728 19.7 / 22.8, 608 / 1216 14.7 / 16.6, k 2560, 144 / 288 5.8 / 6.3; 2 / 1 quads: 128 / 256
+// workgroups of residual rows at k 3072 3.8 / 3.3).
+GemvFn pick_mfma(const Quads& t, bool norm, int* grid) {
   int q = 4;
   if (!t.even(t.groups(4))) q = t.silu || t.groups(2) >= t.cus ? 2 : 1;
-  *threads = nw * kWave;
   *grid = t.groups(q);
-  switch (nw == 4 ? (k <= 512 ? 1 : 2) : 10 * ((k + 1023) / 1024)) {  // chunks per wave (mfma_route: no k in 1025..2048)
-    case 1: return pick_mfma_q<4, 1>(q, epi, norm);
-    case 2: return pick_mfma_q<4, 2>(q, epi, norm);
-    case 30: return pick_mfma_q<8, 3>(q, epi, norm);
-    case 40: return pick_mfma_q<8, 4>(q, epi, norm);
-    default: return nullptr;
-  }
+  return t.k <= 3072 ? pick_mfma_q<3>(q, t.silu, norm) : pick_mfma_q<4>(q, t.silu, norm);  // chunks per wave
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -1010,10 +990,10 @@ __attribute__((visibility("default"))) int bz_gemv(const bz_gemv_args* a, hipStr
   const int rc = bz::device_cu_count(&cus);
   if (rc != BZ_OK) return rc;
   const Quads quads = quads_of(a->k, p.n0, p.n1, ntot - p.n0 - p.n1, a->epilogue == BZ_GEMV_SILU_MUL, cus);
-  if (mfma_route(a->m, a->k, ntot, a->epilogue, quads)) {
-    GemvFn mf = pick_mfma(a->k, quads, a->epilogue, a->norm_weight != nullptr, &bthreads, &bgrid);
+  if (mfma_route(a->m, a->k, a->epilogue, quads)) {
+    GemvFn mf = pick_mfma(quads, a->norm_weight != nullptr, &bgrid);
     if (mf == nullptr) return BZ_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL(mf, dim3(bgrid), dim3(bthreads), 0, stream, p.w0, p.w1, p.w2, p.n0, p.n1, p.ntot,
+    hipLaunchKernelGGL(mf, dim3(bgrid), dim3(kMfmaWaves * kWave), 0, stream, p.w0, p.w1, p.w2, p.n0, p.n1, p.ntot,
                        p.k | a->m << 24, p.x, p.ldx, p);
     return hipGetLastError() == hipSuccess ? BZ_OK : BZ_ERR_LAUNCH;
   }

@@ -669,9 +669,12 @@ __device__ __forceinline__ void consume_tile(Tile<PPT>& t, const uint4 (&qp)[G],
 
 // ------------------------------------------------------------------- tiles on the matrix cores (groups of 4 and 8)
 
-// Groups of 8 always; groups of 4 but in the fused step with lengths (the backbone's decode step): a difference of
-// rounding in one layer's attention travels through every later layer of a step (28 layers: 1.7% in the logits from 1e-5 in
-// each call), and a step's results stay what they were, bit for bit.
+// Groups of 8 always; groups of 4 but in the fused call with lengths, the one a backbone step makes. The two paths sum in
+// another order, a last-bit difference per call that every later layer's roundings carry on: 120 random steps of 2 to 12
+// layers, most of groups of 4, differed between the paths by up to 1.45% of the logits, 7 of them by more than the 1% a step
+// is held to against its earlier outputs, with the same error against 64 bits (0.6 to 1.7%) on both sides. The matrix tiles
+// would save 3 to 15% of that call (2 rows x 8 kv heads x 500 / 1024 / 4096 positions 6.69 / 7.33 / 11.9 us, 6.52 / 6.83 /
+// 10.1), 1 to 4% of such a step. Groups of 8 save 25 to 45% of the call and take them.
 constexpr bool use_mfma(int G, int MK, bool FUSED) { return G == 8 || (G == 4 && !(FUSED && MK == BZ_MASK_NONE)); }
 // A chunk of one or two of the vector path's one-position tiles ends before the matrix tiles' LDS hand-over of 3 G columns
 // pays (G 4, no mask, one split, us per call over 9 / 17 / 32 / 64 positions, vector / matrix: D 128 3.10 / 3.40, 3.42 /
