@@ -35,6 +35,7 @@ NAME = "mi355_decode"
 EAGER_NAME = "mi355_eager"   # eager_attention alone, for reference runs of a model on the GPU
 calls = {"hip": 0, "eager": 0}
 _native = None   # the native binding's hf(): the route's checks and the call in one, once a call has taken the route
+_native_devices: set = set()   # the devices it may run on: those on which a call has taken the route
 
 _SUPPORTED_D = (64, 128)
 _SUPPORTED_G = (1, 2, 4, 8)
@@ -123,9 +124,10 @@ def mi355_decode_attention(module, query: torch.Tensor, key: torch.Tensor, value
         # the query row's mask ([B, 1, 1, S] at decode already: no slicing view to build)
         mask = attention_mask if attention_mask.size(2) == 1 else attention_mask[:, :, -1:, :]
         gqa_decode_masked(query, key, value, mask, scaling, out)
-    if _native is None and not torch.compiler.is_compiling():
+    if (_native is None or query.device.index not in _native_devices) and not torch.compiler.is_compiling():
         eager = kernels.eager()
         eager.allow_device(query.device.index)
+        _native_devices.add(query.device.index)
         _native = eager.hf
     return out, None
 

@@ -82,3 +82,31 @@ def test_install_declines_other_gpus(monkeypatch, capsys):
     assert "not installed: Fake GPU" in capsys.readouterr().out
     q = torch.zeros(1, 4, 1, 64, dtype=torch.bfloat16)
     assert not hf_attention._hip_route(None, q, q, q, None, 0.0)
+
+
+def test_native_form_is_bound_on_every_device(monkeypatch):
+    """Layers on several GPUs: the first call on each device goes the Python way and allows the native form there, the
+    next ones take it. (The query, the kernels and the binding are stand-ins.)"""
+    import types
+
+    from breeze_tts_2_flash_amd import kernels
+
+    allowed, native, python = set(), [], []
+
+    def hf(q, k, v, mask, scaling):
+        if q.device.index not in allowed:
+            return None
+        native.append(q.device.index)
+        return mask
+
+    monkeypatch.setattr(hf_attention, "_native", None)
+    monkeypatch.setattr(hf_attention, "_native_devices", set())
+    monkeypatch.setattr(hf_attention, "_hip_route", lambda *a: True)
+    monkeypatch.setattr(hf_attention, "gqa_decode_masked", lambda q, *a: python.append(q.device.index))
+    monkeypatch.setattr(kernels, "eager", lambda: types.SimpleNamespace(allow_device=allowed.add, hf=hf))
+    mask, mod = torch.zeros(1, 1, 1, 9), types.SimpleNamespace(training=False)
+    monkeypatch.setattr(torch, "empty", lambda *a, **kw: mask)
+    for i in (0, 1, 0, 1, 1):
+        q = types.SimpleNamespace(shape=(1, 4, 1, 64), device=torch.device("cuda", i))
+        hf_attention.mi355_decode_attention(mod, q, None, None, mask)
+    assert python == [0, 1] and native == [0, 1, 1]
