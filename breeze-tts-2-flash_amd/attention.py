@@ -64,8 +64,7 @@ def workspace_bytes(batch: int, num_q_heads: int, num_kv_heads: int, head_dim: i
 
 
 def default_splits(batch: int, num_kv_heads: int, head_dim: int, capacity: int, max_seq_len: int = 0) -> int:
-    """Split count the library picks when num_splits=0 (needs a current device for its CU count); groups of 4 and 8 q
-    heads per kv head may run fewer in batches of more than three rows (bz_gqa_decode_default_splits)."""
+    """Split count the library picks when num_splits=0 (needs a current device for its CU count)."""
     n = ctypes.c_int32(0)
     kernels.check(kernels.load().bz_gqa_decode_default_splits(batch, num_kv_heads, head_dim, capacity, max_seq_len,
                                                                ctypes.byref(n)), "bz_gqa_decode_default_splits")

@@ -124,13 +124,13 @@ int most_splits_for(int64_t units, int D, int len, int cus) {
 //     42.8, 32 45.5, 128 50.7).
 //   - More than three rows are a server's batch, whose lengths differ: two rounds (or three where they divide the row
 //     better and the merge still reads its partials in one batch) even the CUs out, as long as a chunk keeps kMaxChunk
-//     positions (12 rows: 5 splits 16.1, 8 13.8; 16 rows of 512: 2 splits 9.3, 4 9.9), and chunks of two kMaxChunk, however
-//     many rounds that makes. Time against one split per kMaxChunk positions, mean over 16 draws of lengths up to the
-//     capacity / all of that length: 16 rows of 2048 (8 splits): 4 splits 0.99 / 0.97, 6 1.02 / 0.98, 3 1.07 / 1.03; 8 rows
-//     of 4096 (16): 8 splits 0.99 / 0.97, 6 1.08 / 1.03; 14 rows of 4096: 8 splits 0.99 / 0.99, 4 1.02 / 0.96; 20 of 3000
-//     (12): 6 splits 1.01 / 0.94, 3 1.04 / 0.91; 32 of 4096: 8 splits 1.03 / 0.98, 2 1.10 / 0.93. Single draws spread by
-//     10% around these means. The matrix tiles (matrix: groups of 4 and 8) pay more per chunk and stop at the two rounds:
-//     16 rows, G 4, 4096 positions: 4 splits 0.94 / 0.92, 8 0.97 / 0.98.
+//     positions (16 rows of 128..2048: 2 splits 20.7, 4 18.6, 8 19.6; 12: 5 splits 16.1, 8 13.8; 8 of 500..8192: 4 splits
+//     38.6, 8 33.9, 32 34.4; but 16 rows of 512: 2 splits 9.3, 4 9.9). Against one split per kMaxChunk positions, over 220
+//     random batches of up to 32768 positions, half of equal lengths, half spread between a random bound and the longest:
+//     0.91 of the time in the mean and 1.01 at worst, 0.93 and 1.06. Lengths spread wider, from a sixteenth of the longest
+//     up, even out less where that leaves a row few splits (mean of 16 draws: 16 rows of 2048 at 4 splits 0.99, 20 of 3000
+//     at 3 1.04, 32 of 4096 at 2 1.10); four rounds or chunks of at most 512 there cost the others more (0.925 and 0.976
+//     over the 220, where this rule has 0.921).
 //   - Past kMergeBatch splits the merge takes a second batch of partials: worth it up to two batches for chunks of 32 KB
 //     of K+V (1 row of 2048: 16 splits 6.61, 32 6.28; of 4096: 8.24, 7.50; 2 kv heads, G 4, 1000 positions: 16 splits
 //     5.43, 32 6.03), and beyond for chunks of 128 KB (1 kv head x 8192: 16 splits 10.7, 32 8.0, 256 13.7). Never a little
@@ -138,7 +138,7 @@ int most_splits_for(int64_t units, int D, int len, int cus) {
 //     6.14; 2 kv heads, G 4: 6.67, 6.22; 1 row x 1 kv head 5.97, 5.63).
 //   - Rows of up to twice kOneSplitBytes are not split where the rows alone take half of the CUs (16 rows of 200: 1 split
 //     6.09, 2 7.00; 8 such rows: 5.72, 6.39).
-int default_splits_for(int rows, int NKV, int D, int len, int cus, bool matrix) {
+int default_splits_for(int rows, int NKV, int D, int len, int cus) {
   constexpr int kMergeBatch = 16, kPairRows = 3;
   const int64_t units = (int64_t)rows * NKV;
   auto raised = [&](int s, int kb) {  // to chunks of kb KB of K+V, rounded up, where more than s whole ones fit
@@ -152,7 +152,6 @@ int default_splits_for(int rows, int NKV, int D, int len, int cus, bool matrix) 
     int two = (int)(2 * cus / units);
     const int three = (int)(3 * cus / units);
     if (three <= kMergeBatch && 3 * two < 2 * three) two = three;
-    if (!matrix && two < (by_len + 1) / 2) two = (by_len + 1) / 2;
     const int longest = s > by_len ? s : by_len;
     s = two < longest ? two : longest;
   }
@@ -195,8 +194,7 @@ int check_sizes(int B, int NH, int NKV, int D, int cap) {
 int tokens_of(const bz_gqa_decode_args* a) { return a->tokens_per_row > 1 ? a->tokens_per_row : 1; }
 int rows_of(const bz_gqa_decode_args* a) { return a->batch * tokens_of(a); }
 
-// matrix: the call runs on the matrix tiles (use_mfma).
-int resolve_splits(const bz_gqa_decode_args* a, bool matrix, int* splits) {
+int resolve_splits(const bz_gqa_decode_args* a, int* splits) {
   if (a->num_splits < 0 || a->num_splits > kMaxSplits) return BZ_ERR_SHAPE;
   if (a->num_splits > 0) {
     *splits = a->num_splits;
@@ -206,7 +204,7 @@ int resolve_splits(const bz_gqa_decode_args* a, bool matrix, int* splits) {
   const int rc = device_cus(&cus);
   if (rc != BZ_OK) return rc;
   *splits = default_splits_for(rows_of(a), a->num_kv_heads, a->head_dim, effective_len(a->capacity, a->max_seq_len),
-                               cus, matrix);
+                               cus);
   return BZ_OK;
 }
 
@@ -325,9 +323,8 @@ int launch(const bz_gqa_decode_args* a, hipStream_t stream, const int32_t* seq_l
   // the split kernels built without a mask take each row's range from seq_lens alone
   if (mask_kind == BZ_MASK_NONE && seq_lens == nullptr) return BZ_ERR_NULL;
   if (seq_lens != nullptr && wave_route(a, mask_kind, f)) return launch_wave(a, stream, seq_lens, kv_start);
-  const bool matrix = use_mfma(G, mask_kind, f != nullptr);
   int splits = 0;
-  int rc = resolve_splits(a, matrix, &splits);
+  int rc = resolve_splits(a, &splits);
   if (rc != BZ_OK) return rc;
   WsLayout ws;
   char* wsb = nullptr;
@@ -358,6 +355,7 @@ int launch(const bz_gqa_decode_args* a, hipStream_t stream, const int32_t* seq_l
   int chunk = (len + splits - 1) / splits;
   if (chunk < min_chunk) chunk = min_chunk;
   const int nt = kSplitThreads;
+  const bool matrix = use_mfma(G, mask_kind, f != nullptr);
   const int ppt = matrix && !vector_short(G, mask_kind, f != nullptr, splits, len) ? kMatrix : ppt_for(D, chunk, nt);
   SplitFn split_fn = pick_split(D, G, mask_kind, ppt, nt, f != nullptr);
   CombineFn comb_fn = pick_combine(D, G, matrix);
@@ -598,7 +596,7 @@ __attribute__((visibility("default"))) int bz_gqa_decode_default_splits(int32_t 
   int cus = 0;
   const int rc = device_cus(&cus);
   if (rc != BZ_OK) return rc;
-  *num_splits = default_splits_for(batch, num_kv_heads, head_dim, effective_len(capacity, max_seq_len), cus, false);
+  *num_splits = default_splits_for(batch, num_kv_heads, head_dim, effective_len(capacity, max_seq_len), cus);
   return BZ_OK;
 }
 

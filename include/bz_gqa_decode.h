@@ -91,8 +91,7 @@ typedef struct bz_gqa_decode_args {
   void* out;
   int64_t out_stride_b, out_stride_h;
   int32_t batch, num_q_heads, num_kv_heads, head_dim, capacity;
-  /* workgroups per (batch, kv head); 0 picks bz_gqa_decode_default_splits(.., max_seq_len or capacity, ..), or fewer
-     (see there) */
+  /* workgroups per (batch, kv head); 0 picks bz_gqa_decode_default_splits(.., max_seq_len or capacity, ..) */
   int32_t num_splits;
   /* expected upper bound of seq_lens - kv_start (0 = capacity); only steers the default tiling */
   int32_t max_seq_len;
@@ -137,11 +136,9 @@ int bz_gqa_decode_noalloc(const bz_gqa_decode_args* args, hipStream_t stream);
 int bz_gqa_decode_workspace_size(int32_t batch, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
                                  int32_t capacity, int32_t num_splits, int32_t max_seq_len, size_t* bytes);
 
-/* The split count the decode entry points use when num_splits == 0 (device CU count, sizes; with tokens_per_row T > 1
-   pass batch * T): exactly this for groups of 1 and 2 q heads per kv head, at most this for groups of 4 and 8, which run
-   fewer, longer splits in batches of more than three rows whose chunks are longer than 512 positions. A workspace sized
-   for this count serves every such call. No counterpart in the reference, which fixes 64-position chunks at compile time
-   (bb_attn.cu:28, :382). */
+/* The split count bz_gqa_decode uses when num_splits == 0 (device CU count, sizes; with tokens_per_row T > 1 pass
+   batch * T). No counterpart in the
+   reference, which fixes 64-position chunks at compile time (bb_attn.cu:28, :382). */
 int bz_gqa_decode_default_splits(int32_t batch, int32_t num_kv_heads, int32_t head_dim, int32_t capacity,
                                  int32_t max_seq_len, int32_t* num_splits);
 

@@ -25,7 +25,6 @@ CASES = [
     (4, 16, 8, 128, 1024, 8),     # a batch of short rows stays at one round
     (16, 16, 8, 128, 2048, 4),    # two rounds
     (12, 8, 8, 64, 2048, 8),      # three rounds divide the row better
-    (20, 8, 8, 64, 2100, 5),      # more rounds, for chunks of at most 512 positions
     (16, 16, 8, 128, 256, 1),     # half of the CUs taken by the rows alone, 128 KB a row: no split
     (15, 16, 8, 128, 256, 2),     # just below half of the CUs
     (16, 16, 8, 128, 264, 2),     # just above 128 KB
@@ -44,21 +43,6 @@ def test_default_split_count(device, B, NH, NKV, D, cap, splits):
     out = gqa_decode(g.q, g.k, g.v, g.seq_lens, g.scale, kv_start=st.to(device))
     torch.cuda.synchronize()
     assert_close(out.float().cpu().numpy(), oracle(w, kv_start=starts), f"B={B} NKV={NKV} cap={cap}")
-
-
-def test_matrix_tiles_stop_at_two_rounds(device):
-    """Groups of 4 over the same 20 rows of 2100 positions: 3 splits (480 workgroups), in a workspace sized for the queried
-    count of 5."""
-    if torch.cuda.get_device_properties(device).multi_processor_count != 256:
-        pytest.skip("the counts are those of 256 CUs")
-    B, NH, NKV, D, cap = 20, 32, 8, 64, 2100
-    w, _ = rand_case(7, B, NH, NKV, D, cap, [cap - 97 * b for b in range(B)])
-    g = w.to(device)
-    ws = torch.zeros(workspace_bytes(B, NH, NKV, D, cap, default_splits(B, NKV, D, cap)), dtype=torch.uint8, device=device)
-    outs = [gqa_decode(g.q, g.k, g.v, g.seq_lens, g.scale, num_splits=n, workspace=ws) for n in (0, 3)]
-    torch.cuda.synchronize()
-    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
-    assert_close(outs[0].float().cpu().numpy(), oracle(w), "G 4, 20 rows")
 
 
 def test_static_scratch_refuses_by_the_largest_default(device):
