@@ -907,13 +907,13 @@ GemvFn pick_mfma_q(int q, bool silu, bool norm) {
   return pick_mfma_epi<TR, 1>(silu, norm);
 }
 
-// Quads per workgroup: four where their grid is even, else two, or one where two leave CUs without a workgroup (us per call,
-// 4 / 2 quads: plain at k 4096, 384 / 768 workgroups 12.9 / 12.0, k 3584, 640 / 1280 16.0 / 17.6; gate / up at k 2976, 620 /
-// 1240 13.5 / 12.6, k 3328, 864 / 1728 19.7 / 22.8, 608 / 1216 14.7 / 16.6, k 2560, 144 / 288 5.8 / 6.3; 2 / 1 quads: 128 / 256
-// workgroups of residual rows at k 3072 3.8 / 3.3).
+// Quads per workgroup: four where their grid is even, else two, or one where all of those fit one round (us per call, 4 / 2
+// quads: plain at k 4096, 384 / 768 workgroups 12.9 / 12.0, k 3584, 640 / 1280 16.0 / 17.6; gate / up at k 2976, 620 / 1240
+// 13.5 / 12.6, k 3328, 864 / 1728 19.7 / 22.8, 608 / 1216 14.7 / 16.6, k 2560, 144 / 288 5.8 / 6.3; 2 / 1 quads, plain at k
+// 3072, M = 3: 128 / 256 workgroups 4.7 / 4.2, 144 / 288 4.7 / 5.3).
 GemvFn pick_mfma(const Quads& t, bool norm, int* grid) {
   int q = 4;
-  if (!t.even(t.groups(4))) q = t.silu || t.groups(2) >= t.cus ? 2 : 1;
+  if (!t.even(t.groups(4))) q = t.silu || t.groups(1) > t.cus ? 2 : 1;
   *grid = t.groups(q);
   return t.k <= 3072 ? pick_mfma_q<3>(q, t.silu, norm) : pick_mfma_q<4>(q, t.silu, norm);  // chunks per wave
 }

@@ -37,7 +37,9 @@ def test_gateup(device, M, K, N):
                                     (3, 3000, (5, 1, 2)), (4, 4096, (1024, 512, 512)), (3, 4096, (1, 0, 0)),
                                     # four quads a workgroup, ragged segments: one round, two and a half past k = 3072
                                     (4, 2056, (1030, 513, 517)), (3, 3072, (2049, 1022, 1001)), (3, 3584, (5121, 2563, 2553)),
-                                    (4, 2560, (2001, 1603, 1602))])  # two quads
+                                    (4, 2560, (2001, 1603, 1602)),  # two quads
+                                    # one quad a workgroup in a full round, two where those would be more
+                                    (4, 2560, (1000, 11, 9)), (3, 3584, (513, 258, 262))])
 def test_segments(device, M, K, ns, norm):
     rng = np.random.default_rng(M * K + sum(ns))
     x = rand_bits(rng, M, K)
